@@ -34,6 +34,7 @@ struct soc_ctx {
   size_t sample_ws_bytes = 0;
   int* sample_out = nullptr;
   int* sample_host = nullptr;   // pinned host copy of the output block (hipHostMalloc)
+  int* sample_host_dev = nullptr;  // the address kernels use for it
   // pinned host words a decode step's readback kernel writes (next token, wait error, token id error), with the
   // address kernels use for them
   int32_t* readback = nullptr;

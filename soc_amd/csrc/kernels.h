@@ -150,8 +150,14 @@ constexpr size_t kSampleTreeBytes = 48 * 1024;
 // Whether a row of V logits at this k is searched on the device (k <= kSampleMaxK and the lists fit).
 bool sample_device_fits(int V, int k);
 // Device workspace bytes for a row of V logits; zero-filled when allocated (its first word is an arrival counter
-// that every k = 1 search leaves at zero).
+// that every launch_sample_head leaves at zero).
 size_t sample_ws_bytes(int V);
+// The search in one launch, for rows whose k largest values of row / t differ (and any row at k = 1): out[0] = k,
+// out[1] = 0, then k (index, bits of its raw logit) pairs from the largest down. out[1] = 1: the row holds a NaN;
+// out[1] = 2: equal values among the k largest, launch_sample_topk has to search. out takes 2 + 2 k words, in device or
+// pinned host memory. Requires sample_head_fits(V, k).
+bool sample_head_fits(int V, int k);
+hipError_t launch_sample_head(const float* row, int V, float t, int k, void* ws, int* out, hipStream_t s);
 // Finds the candidates that std::partial_sort(top k of row / t) over 0..V-1 moves into its heap, in index order:
 // out[0] = count, out[1] = NaN seen, then for j < min(count, max_out): out[2 + 2 j] = index,
 // out[3 + 2 j] = the bits of its raw logit. Requires sample_device_fits(V, k).

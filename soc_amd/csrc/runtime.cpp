@@ -2743,26 +2743,43 @@ int soc_sample_topk(soc_ctx* ctx, const float* row, int32_t vocab, int32_t top_k
     if (ctx->sample_host == nullptr &&
         (e = hipHostMalloc(reinterpret_cast<void**>(&ctx->sample_host), kOutInts * sizeof(int))) != hipSuccess)
       return hip_fail(e, "hipHostMalloc sampler output");
-    if ((e = soc::launch_sample_topk(row, vocab, t, k, ctx->sample_ws, ctx->sample_out, kMaxOut, s)) != hipSuccess)
-      return hip_fail(e, "sampler launch");
-    // the head of the block first (it holds every candidate of a typical row), the rest only when needed
-    constexpr int kHead = 512;
+    if (ctx->sample_host_dev == nullptr &&
+        (e = hipHostGetDevicePointer(reinterpret_cast<void**>(&ctx->sample_host_dev), ctx->sample_host, 0)) !=
+            hipSuccess)
+      return hip_fail(e, "hipHostGetDevicePointer");
+    // one launch that writes its candidates into pinned host memory; the general search and its copies only for a row
+    // with equal values among its k largest
     const int* out = ctx->sample_host;
-    if ((e = hipMemcpyAsync(ctx->sample_host, ctx->sample_out, (2 + 2 * kHead) * sizeof(int), hipMemcpyDeviceToHost,
-                            s)) != hipSuccess)
-      return hip_fail(e, "hipMemcpyAsync sampler");
-    if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "sampler");
-    const int n = out[0];
-    if (out[1] != 0 || n > kMaxOut || n < k) {
-      whole_row = true;  // NaN logits, or more candidates than the output block holds: the reference's full sort
-    } else {
-      if (n > kHead) {
+    int n = 0, flag = 2;
+    if (soc::sample_head_fits(vocab, k)) {
+      if ((e = soc::launch_sample_head(row, vocab, t, k, ctx->sample_ws, ctx->sample_host_dev, s)) != hipSuccess)
+        return hip_fail(e, "sampler launch");
+      if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "sampler");
+      n = out[0];
+      flag = out[1];
+    }
+    if (flag == 2) {
+      if ((e = soc::launch_sample_topk(row, vocab, t, k, ctx->sample_ws, ctx->sample_out, kMaxOut, s)) != hipSuccess)
+        return hip_fail(e, "sampler launch");
+      // the head of the block first (it holds every candidate of a typical row), the rest only when needed
+      constexpr int kHead = 512;
+      if ((e = hipMemcpyAsync(ctx->sample_host, ctx->sample_out, (2 + 2 * kHead) * sizeof(int), hipMemcpyDeviceToHost,
+                              s)) != hipSuccess)
+        return hip_fail(e, "hipMemcpyAsync sampler");
+      if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "sampler");
+      n = out[0];
+      flag = out[1];
+      if (flag == 0 && n > kHead && n <= kMaxOut) {
         if ((e = hipMemcpyAsync(ctx->sample_host + 2 + 2 * kHead, ctx->sample_out + 2 + 2 * kHead,
                                 static_cast<size_t>(n - kHead) * 2 * sizeof(int), hipMemcpyDeviceToHost, s)) !=
             hipSuccess)
           return hip_fail(e, "hipMemcpyAsync sampler");
         if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "sampler");
       }
+    }
+    if (flag != 0 || n > kMaxOut || n < k) {
+      whole_row = true;  // NaN logits, or more candidates than the output block holds: the reference's full sort
+    } else {
       idx.resize(n);
       vals.resize(n);
       for (int j = 0; j < n; ++j) {

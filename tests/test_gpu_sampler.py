@@ -119,3 +119,31 @@ def test_sample_topk_rejects_row_past_its_allocation(gpu_ctx):
             S.sample_topk(gpu_ctx, p, 1_000_000, 5, 1.0)
     finally:
         gpu_ctx.free(p)
+
+
+@pytest.mark.parametrize("k", [2, 50, 64])
+def test_sample_topk_one_launch_search(gpu_ctx, oracle_mod, k):
+    """The one-launch search of rows whose k largest values differ, at the edges of its groups (16 values, 64 from
+    V = 32768), of a block's 2048 values and of the group maxima one block ranks, with every value in one group; and
+    equal values straddling rank k (which only the general search orders) or just past it (which changes nothing)."""
+    rng = np.random.default_rng(k)
+    sizes = [k, k + 1, 16 * k - 1, 16 * k, 2047, 2048, 2049, 32767, 32768, 151936, 151937]
+    for v in sizes + ([524288, 524289] if k <= 20 else []):
+        row = rng.permutation(v).astype(np.float32) - v / 3
+        packed = np.sort(row)[::-1].copy()          # the k largest side by side, one -inf, both zeros
+        packed[-1] = -np.inf
+        at_k, past_k = row.copy(), row.copy()
+        order = np.argsort(-row)
+        if v > k + 1:
+            at_k[order[k]] = row[order[k - 1]]      # ranks k and k + 1 equal
+            past_k[order[k]] = row[order[k + 1]]    # ranks k + 1 and k + 2 equal
+        for what, r in (("distinct", row), ("packed", packed), ("tie at k", at_k), ("tie past k", past_k)):
+            p = gpu_ctx.upload(r)
+            try:
+                for t in (1.0, 0.7):
+                    tok, ids, vals = S.sample_topk(gpu_ctx, p, v, k, t)
+                    rtok, rids, rvals = oracle_mod.sample_topk(r, t, k)
+                    assert tok == rtok and np.array_equal(ids, rids), f"{what}, V {v}, temperature {t}"
+                    assert np.array_equal(vals.view(np.uint32), rvals.view(np.uint32))
+            finally:
+                gpu_ctx.free(p)
