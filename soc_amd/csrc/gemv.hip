@@ -308,20 +308,19 @@ __global__ __launch_bounds__(256) void k_lm_head_argmax(LmHeadArgs a) {
   }
 }
 
-// Group-quantized GEMV/skinny GEMM: y[m][n] = sum_g scale[n][g] * sum_{k in group g} x[m][k] * code[n][k], with
-// groups of 64 along K (the product per element is w = float(code) * float(scale), dequant_group's contract).
-// BITS = 8: codes int8 [N][K]; BITS = 4: two's complement nibbles, even k in the low nibble, [N][K/2].
+// Group-quantized matmul kernels of soc_qmm beyond qrows.hip: y[m][n] = sum_g scale[n][g] * sum_{k in group g}
+// x[m][k] * code[n][k], with groups of 64 along K (the product per element is w = float(code) * float(scale),
+// dequant_group's contract). BITS = 8: codes int8 [N][K]; BITS = 4: two's complement nibbles, even k in the low nibble,
+// [N][K/2].
 //
-// Each lane streams 16-byte chunks of a row's codes (16 int8 or 32 int4 codes; a chunk never crosses a scale
-// group). The codes become exact fp16 pairs without per-code conversions: the biased code (code + 128, or the
-// nibble + 8) is placed in the low mantissa bits of 1024.0 (fp16 0x64xx) by one byte permute (int8) or one
-// mask-xor (int4), and one packed fp16 subtract of 1152 (or 1032) leaves the code itself (int4 nibbles in bits
-// 4..7: one packed fma by 1/16 minus 72, so that half the nibbles need no shift). v_dot2_f32_f16 then
-// accumulates code pairs times fp16 activation pairs in fp32 (products exact), and one fma per chunk applies the
-// group scale. The activations are staged once per block in LDS as fp16 pairs in the order the codes unpack
-// (int4: k and k + 4 of each group of 8). L lanes share a row (64, or 32 / 16 for short rows) and each lane
-// keeps RR rows in flight: 4 rows per wave for tall matrices, one row per lane group when fewer than 4096 rows
-// would leave most SIMDs idle.
+// k_qmm (two rows of tall matrices, and operands off 16-byte alignment): each lane streams 16-byte chunks of a row's codes (16 int8 or 32 int4 codes; a
+// chunk never crosses a scale group). The codes become exact fp16 pairs without per-code conversions: the biased code
+// (code + 128, or the nibble + 8) is placed in the low mantissa bits of 1024.0 (fp16 0x64xx) by one byte permute (int8)
+// or one mask-xor (int4), and one packed fp16 subtract of 1152 (or 1032) leaves the code itself (int4 nibbles in bits
+// 4..7: one packed fma by 1/16 minus 72, so that half the nibbles need no shift). v_dot2_f32_f16 then accumulates code
+// pairs times fp16 activation pairs in fp32 (products exact), and one fma per chunk applies the group scale. The
+// activations are staged once per block in LDS as fp16 pairs in the order the codes unpack (int4: k and k + 4 of each
+// group of 8). L lanes share a row (64, or 32 / 16 for short rows) and each lane keeps RR rows in flight.
 namespace {
 typedef _Float16 qh2 __attribute__((ext_vector_type(2)));
 typedef _Float16 sk_qh8 __attribute__((ext_vector_type(8)));
@@ -873,11 +872,20 @@ bool qmm_mfma_supported(const QmmArgs& a, int bits) {
           reinterpret_cast<uintptr_t>(a.scales)) % 16 == 0;
 }
 
+// Which kernel a soc_qmm call takes, by shape (us measured on MI355X, both sides):
+//  - one row: k_qgemv. At least as fast as the kernel it replaced over 1024 .. 151936 x 1024 .. 9728 (4 to 15 % where the
+//    matrix is tall, up to 33 % on long rows).
+//  - 2 to 8 rows of a tall matrix (N >= 16384) with whole chunks of K (k_qmm_mfma's form): k_qmm_mfma. 151936 x 1024
+//    x 8: int4 17.6 against 26.8 for k_qrows, int8 28.4 against 32.9.
+//  - two rows, otherwise: the dot products of k_qmm where the matrix is tall enough to stream (int8 12000 x 3008 10.6
+//    against 12.2; int4 60000 x 1536 17.1 against 18.5; 40000 x 8192 50.7 against 69.2), k_qrows elsewhere (int4 2048
+//    < K <= 5120 at any height: 19456 x 2560 10.9 against 14.2; below 8192 rows: 2560 x 4096 5.9 against 7.0; below
+//    4096 rows also for longer K: 1024 x 6144 8.0 against 8.9).
+//  - four or eight rows: k_qrows (12000 x 3008 int4 x 8 9.8 against 23.4 for the dot products; int8 13.1 against 21.7).
+//  - operands off 16-byte alignment: k_qmm, or k_qmm_short for rows of fewer than 16 chunks.
+// SOC_QMM=mfma takes k_qmm_mfma wherever it applies (the parity tests run it on the short shapes too).
 hipError_t launch_qmm(const QmmArgs& a, int bits, hipStream_t s) {
   const char* mode = std::getenv("SOC_QMM");
-  // matrix cores for tall matrices (the LM head); the dot-product kernel keeps the short ones, where a 128-row
-  // block per 16 waves would leave most of the chip idle (SOC_QMM=mfma takes the MFMA kernel wherever it applies:
-  // the parity tests run it on the short shapes too)
   const bool force_mfma = mode != nullptr && std::strcmp(mode, "mfma") == 0;
   if (qmm_mfma_supported(a, bits) && (force_mfma || a.N >= 16384)) {
     const size_t lds = static_cast<size_t>(16) * (a.K + 8) * sizeof(f16);
@@ -888,10 +896,22 @@ hipError_t launch_qmm(const QmmArgs& a, int bits, hipStream_t s) {
     else hipLaunchKernelGGL(k_qmm_mfma<4>, grid, block, lds, s, a);
     return hipGetLastError();
   }
+  QRowsArgs q{};
+  q.xh = a.x;
+  q.codes = a.codes;
+  q.scales = a.scales;
+  q.y = a.y;
+  q.M = a.M;
+  q.N = a.N;
+  q.K = a.K;
   const int nch = a.K / (bits == 8 ? 16 : 32);  // 16-byte chunks per row
+  const bool rows2 = (bits == 4 && a.K > 2048 && a.K <= 5120) || (a.N < 8192 && (a.K <= 5120 || a.N < 4096));
+  const bool dot = a.M == 2 && nch >= 16 && !rows2;
+  if (qrows_supported(q, bits) && !dot) return launch_qrows(q, bits, EPI_STORE, s);
+  const dim3 block(256);
   if (nch < 16) {
     const size_t lds = static_cast<size_t>(a.M) * a.K * sizeof(float);
-    const dim3 grid(gemv_grid(a.N, 2)), block(256);
+    const dim3 grid(gemv_grid(a.N, 2));
 #define SOC_QMM_SHORT(B, MM)                                                       \
     if (bits == B && a.M == MM) {                                                 \
       hipLaunchKernelGGL((k_qmm_short<B, MM>), grid, block, lds, s, a);            \
@@ -908,7 +928,7 @@ hipError_t launch_qmm(const QmmArgs& a, int bits, hipStream_t s) {
   const size_t lds = static_cast<size_t>(a.M) * a.K * sizeof(f16);
   const int waves = (a.N + rows_per_wave - 1) / rows_per_wave;
   const int blocks = std::min((waves + 3) / 4, 2048);
-  const dim3 grid(std::max(blocks, 1)), block(256);
+  const dim3 grid(std::max(blocks, 1));
 #define SOC_QMM_CASE(B, MM, LL)                                                                    \
   if (bits == B && a.M == MM && L == LL) {                                                        \
     if (tall) hipLaunchKernelGGL((k_qmm<B, MM, LL, 4 * LL / 64>), grid, block, lds, s, a);         \

@@ -49,6 +49,23 @@ struct QmmArgs {
   int M, N, K;
 };
 hipError_t launch_qmm(const QmmArgs& a, int bits, hipStream_t s);
+// The same products for 1 <= M <= 8 rows on matrix cores, with a decode projection's neighbours fused in
+// (qrows.hip). Activations: xh (fp16 [M][K]), or x (fp32, rounded to fp16), or RMSNorm(x) with `gain` (rounded).
+//   EPI_STORE: y = sums (xh, or x with gain). EPI_RESIDUAL: y += sums (xh, or x without gain). EPI_SWIGLU: rows
+//   [0, N / 2) are gate and [N / 2, N) up: yh [M][N / 2] = fp16(silu(gate) * up) (x with gain).
+struct QRowsArgs {
+  const f16* xh;
+  const float* x;
+  const f16* gain;
+  float eps;
+  const void* codes;
+  const f16* scales;
+  float* y;    // [M][N]
+  f16* yh;
+  int M, N, K;
+};
+bool qrows_supported(const QRowsArgs& a, int bits);
+hipError_t launch_qrows(const QRowsArgs& a, int bits, int epi, hipStream_t s);
 hipError_t launch_dequant(const void* codes, int bits, const f16* scales, int N, int K, float* w, hipStream_t s);
 // The same weights rounded to fp16 (nearest) [N][K], for the prefill GEMMs of a quantized model (K % 64 == 0).
 hipError_t launch_dequant_f16(const void* codes, int bits, const f16* scales, int N, int K, f16* w, hipStream_t s);
@@ -137,11 +154,8 @@ hipError_t launch_decode_readback(const int32_t* state, const int32_t* wait_err,
 // dst[0..n) = src[0..n) for n <= 16 words read from the host at launch (the words travel as kernel arguments).
 hipError_t launch_write_words(int32_t* dst, const int32_t* src, int n, hipStream_t s);
 
-// ---- quantized-model forward steps (qpath.hip) ----
+// y = fp16(x), rounded to nearest even (qpath.hip)
 hipError_t launch_f32_to_f16(const float* x, size_t n, f16* y, hipStream_t s);
-hipError_t launch_add_f32(float* x, const float* y, size_t n, hipStream_t s);  // x += y
-// gu [T][2 I] (gate | up) -> h [T][I] = fp16(silu(gate) * up)
-hipError_t launch_swiglu_f16(const float* gu, int T, int I, f16* h, hipStream_t s);
 
 // ---- sampler: top-k candidates of one logits row (sample.hip) ----
 constexpr int kSampleChunk = 2048, kSampleMaxK = 64;

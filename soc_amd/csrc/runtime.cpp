@@ -92,9 +92,8 @@ struct DecodeWs {
   float* pv = nullptr;
   int *pi = nullptr, *err = nullptr;
   int nblocks = 0;
-  // quantized models: fp16 activation row and fp32 projection output of the per-op decode
+  // quantized models: SwiGLU output row
   f16* qx = nullptr;
-  float* qy = nullptr;
   std::vector<void*> allocs;
 };
 
@@ -108,7 +107,7 @@ struct PrefillWs {
   float* skpart = nullptr;  // split-K partials of the skinny batch projections
   // hi/lo fp16 activation pairs of the prefill projections: p = normed input / attention output, q = SwiGLU output
   soc::f16 *ph = nullptr, *pl = nullptr, *qh = nullptr, *ql = nullptr;
-  // quantized models: fp16 activation rows and fp32 projection outputs of one chunk of kQChunk rows
+  // quantized models: SwiGLU outputs and QKV projections of one chunk of kQChunk rows
   soc::f16* qx = nullptr;
   float* qy = nullptr;
 };
@@ -282,12 +281,7 @@ int ensure_decode_ws(soc_model* m, int cap) {
   SOC_TRY(dev_alloc_t(w.allocs, 64, &w.state));
   SOC_TRY(dev_alloc_t(w.allocs, cap, &w.ring));
   SOC_TRY(dev_alloc_t(w.allocs, 64, &w.ring_pos));
-  {
-    const size_t kmax = std::max({c.hidden_size, m->qd, c.intermediate_size});
-    const size_t nmax = std::max({m->qkv_rows, 2 * c.intermediate_size, c.hidden_size});
-    SOC_TRY(dev_alloc_t(w.allocs, kmax, &w.qx));
-    SOC_TRY(dev_alloc_t(w.allocs, nmax, &w.qy));
-  }
+  SOC_TRY(dev_alloc_t(w.allocs, c.intermediate_size, &w.qx));
   hipError_t e;
   if ((e = hipMemset(w.lm_counter, 0, 64 * sizeof(int))) != hipSuccess) return hip_fail(e, "hipMemset");
   if ((e = hipMemset(w.attn_counters, 0, c.num_key_value_heads * sizeof(int))) != hipSuccess)
@@ -366,13 +360,8 @@ int ensure_prefill_ws(soc_model* m, int rows, int total_len, int logit_rows) {
   SOC_TRY(dev_alloc_t(w.allocs, 1024, &w.lm_idx));
   SOC_TRY(dev_alloc_t(w.allocs, 64, &w.lm_counter));
   SOC_TRY(dev_alloc_t(w.allocs, 64, &w.token));
-  {
-    const size_t kmax = std::max({c.hidden_size, m->qd, c.intermediate_size});
-    const size_t nmax = std::max({m->qkv_rows, 2 * c.intermediate_size, c.hidden_size});
-    SOC_TRY(dev_alloc_t(w.allocs, kQChunk * kmax, &w.qx));
-    SOC_TRY(dev_alloc_t(w.allocs, kQChunk * nmax, &w.qy));
-    if ((e = hipMemset(w.qx, 0, kQChunk * kmax * sizeof(soc::f16))) != hipSuccess) return hip_fail(e, "hipMemset");
-  }
+  SOC_TRY(dev_alloc_t(w.allocs, static_cast<size_t>(kQChunk) * c.intermediate_size, &w.qx));
+  SOC_TRY(dev_alloc_t(w.allocs, static_cast<size_t>(kQChunk) * m->qkv_rows, &w.qy));
   if (const size_t sk = skinny_scratch_floats(m)) {
     SOC_TRY(dev_alloc_t(w.allocs, sk, &w.skpart));
     if ((e = soc::skinny_configure()) != hipSuccess) return hip_fail(e, "skinny kernel attributes");
@@ -430,46 +419,48 @@ soc::AttnArgs attn_args(soc_model* m, soc_kv* kv, int layer) {
   return a;
 }
 
-// y[M][N] = x[M][K] . W^T on the model's group-quantized codes (M in 1, 2, 4, 8).
-hipError_t qmm_rows(const soc_model* m, const soc::f16* x, int M, const uint8_t* codes, const soc::f16* scales, int N,
-                    int K, float* y, hipStream_t s) {
-  soc::QmmArgs q{};
-  q.x = x;
-  q.codes = codes;
-  q.scales = scales;
-  q.y = y;
-  q.M = M;
-  q.N = N;
-  q.K = K;
-  return soc::launch_qmm(q, m->qbits, s);
-}
-
-// One layer of a quantized model on T rows x (fp32 [T][H]) whose attention input comes out of `qkv_out` (rows of
-// [T][qkv_rows], M >= T the projection row count): input RMSNorm -> fp16, QKV projection; the caller's attention
-// writes attn (fp32 [T][qd]); then o projection + residual, post RMSNorm -> fp16, gate/up projection, SwiGLU -> fp16,
-// down projection + residual. `attend` enqueues the attention.
+// One layer of a quantized model on T <= kQChunk rows x (fp32 [T][H]): the QKV projection of RMSNorm(x) into qkv_out
+// ([T][qkv_rows]), the caller's attention (`attend`, writing attn, fp32 [T][qd]), the o projection added to x, SwiGLU of
+// the gate/up projection of RMSNorm(x) into h (fp16 [T][I]), and the down projection added to x. Every projection
+// rounds its input rows to fp16; norms, residuals and SwiGLU are fused into the projections (four launches and the
+// attention; as separate kernels they were eleven, most of them shorter than a launch).
 template <typename Attend>
-int enqueue_layer_q(soc_model* m, int l, float* x, int T, int M, soc::f16* qx, float* qy, float* qkv_out,
-                    const float* attn, Attend attend, hipStream_t s) {
+int enqueue_layer_q(soc_model* m, int l, float* x, int T, soc::f16* h, float* qkv_out, const float* attn, Attend attend,
+                    hipStream_t s) {
   const soc_qwen_config& c = m->cfg;
   const DevLayer& L = m->layers[l];
   const QLayer& Q = m->qlayers[l];
   const int H = c.hidden_size, I = c.intermediate_size;
+  soc::QRowsArgs g{};
+  g.M = T;
+  g.eps = c.rms_norm_eps;
+  auto weights = [&](const uint8_t* codes, const soc::f16* scales, int N, int K) {
+    g.codes = codes;
+    g.scales = scales;
+    g.N = N;
+    g.K = K;
+  };
   hipError_t e;
-  if ((e = soc::launch_rmsnorm_rows(x, T, H, L.in_norm, c.rms_norm_eps, nullptr, qx, nullptr, s)) != hipSuccess)
-    return hip_fail(e, "rmsnorm");
-  if ((e = qmm_rows(m, qx, M, Q.qkv, Q.qkv_s, m->qkv_rows, H, qkv_out, s)) != hipSuccess) return hip_fail(e, "qmm qkv");
+  weights(Q.qkv, Q.qkv_s, m->qkv_rows, H);
+  g.x = x;
+  g.gain = L.in_norm;
+  g.y = qkv_out;
+  if ((e = soc::launch_qrows(g, m->qbits, soc::EPI_STORE, s)) != hipSuccess) return hip_fail(e, "quantized qkv");
   SOC_TRY(attend());
-  if ((e = soc::launch_f32_to_f16(attn, static_cast<size_t>(T) * m->qd, qx, s)) != hipSuccess)
-    return hip_fail(e, "f32 -> f16");
-  if ((e = qmm_rows(m, qx, M, Q.o, Q.o_s, H, m->qd, qy, s)) != hipSuccess) return hip_fail(e, "qmm o");
-  if ((e = soc::launch_add_f32(x, qy, static_cast<size_t>(T) * H, s)) != hipSuccess) return hip_fail(e, "residual");
-  if ((e = soc::launch_rmsnorm_rows(x, T, H, L.post_norm, c.rms_norm_eps, nullptr, qx, nullptr, s)) != hipSuccess)
-    return hip_fail(e, "rmsnorm");
-  if ((e = qmm_rows(m, qx, M, Q.gu, Q.gu_s, 2 * I, H, qy, s)) != hipSuccess) return hip_fail(e, "qmm gate/up");
-  if ((e = soc::launch_swiglu_f16(qy, T, I, qx, s)) != hipSuccess) return hip_fail(e, "swiglu");
-  if ((e = qmm_rows(m, qx, M, Q.down, Q.down_s, H, I, qy, s)) != hipSuccess) return hip_fail(e, "qmm down");
-  if ((e = soc::launch_add_f32(x, qy, static_cast<size_t>(T) * H, s)) != hipSuccess) return hip_fail(e, "residual");
+  weights(Q.o, Q.o_s, H, m->qd);
+  g.x = attn;
+  g.gain = nullptr;
+  g.y = x;
+  if ((e = soc::launch_qrows(g, m->qbits, soc::EPI_RESIDUAL, s)) != hipSuccess) return hip_fail(e, "quantized o");
+  weights(Q.gu, Q.gu_s, 2 * I, H);
+  g.x = x;
+  g.gain = L.post_norm;
+  g.yh = h;
+  if ((e = soc::launch_qrows(g, m->qbits, soc::EPI_SWIGLU, s)) != hipSuccess) return hip_fail(e, "quantized gate/up");
+  weights(Q.down, Q.down_s, H, I);
+  g.x = nullptr;
+  g.xh = h;
+  if ((e = soc::launch_qrows(g, m->qbits, soc::EPI_RESIDUAL, s)) != hipSuccess) return hip_fail(e, "quantized down");
   return SOC_OK;
 }
 
@@ -501,7 +492,7 @@ int enqueue_decode(soc_model* m, soc_kv* kv, int slot, const int32_t* d_slot) {
         const hipError_t ea = soc::launch_attention(a, 1, s);
         return ea == hipSuccess ? SOC_OK : hip_fail(ea, "attention decode");
       };
-      SOC_TRY(enqueue_layer_q(m, l, w.x, 1, 1, w.qx, w.qy, w.qkv, w.attn, attend, s));
+      SOC_TRY(enqueue_layer_q(m, l, w.x, 1, w.qx, w.qkv, w.attn, attend, s));
     }
   } else {
     if ((e = soc::launch_embed(w.state, 1, m->embed, c.hidden_size, w.x, s)) != hipSuccess) return hip_fail(e, "embed");
@@ -1846,7 +1837,6 @@ int prefill_layers_q(soc_model* m, soc_kv* kv, int slot, int n, int pos_off, con
   const int H = c.hidden_size;
   for (int c0 = 0; c0 < n; c0 += kQChunk) {
     const int T = std::min(kQChunk, n - c0);
-    const int M = T <= 1 ? 1 : T <= 2 ? 2 : T <= 4 ? 4 : 8;  // the projection's row count (rows past T unused)
     float* xr = w.x + static_cast<size_t>(c0) * H;
     float* qrow = w.q + static_cast<size_t>(c0) * m->qd;
     float* arow = w.attn + static_cast<size_t>(c0) * m->qd;
@@ -1889,7 +1879,7 @@ int prefill_layers_q(soc_model* m, soc_kv* kv, int slot, int n, int pos_off, con
         e = soc::launch_attention(a, 0, s);
         return e == hipSuccess ? SOC_OK : hip_fail(e, "attention");
       };
-      SOC_TRY(enqueue_layer_q(m, l, xr, T, M, w.qx, w.qy, w.qy, arow, attend, s));
+      SOC_TRY(enqueue_layer_q(m, l, xr, T, w.qx, w.qy, arow, attend, s));
     }
   }
   return SOC_OK;

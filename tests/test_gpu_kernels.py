@@ -115,3 +115,31 @@ def test_dequant_bit_exact(gpu_ctx, oracle_mod, bits):
             ctx.free(p)
     ref = oracle_mod.dequant_group(codes, bits, scales, n, k)
     assert np.array_equal(w.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("n,k", [
+    (1, 64), (17, 64), (15, 128), (33, 192),          # one group; an odd number of groups (a half-empty int4 unit)
+    (100, 1088), (16, 2112), (63, 3136), (48, 4160),  # past each count of code loads a wave keeps (1, 2, 3, 4 of 1024 /
+    (20, 5120),                                       # 512 k), the longest row of eight
+    (8191, 320), (8192, 320), (9001, 704),            # either side of the two-row rule's height
+    (32768, 1024), (40001, 1920), (33000, 960),       # tall: fewer waves over K
+])
+@pytest.mark.parametrize("m", [1, 2, 4, 8])
+def test_qmm_row_kernels_match_oracle(gpu_ctx, oracle_mod, bits, m, n, k):
+    """soc_qmm by shape: remainders of the row kernels' tiles, code units and wave splits, against the oracle's matmul
+    within the summation bound. Aligned operands, and activations one half off 16-byte alignment."""
+    ctx = gpu_ctx
+    codes, scales, x = _qmm_inputs(n, k, bits, m)
+    ref = oracle_mod.qmm_group(x, codes, bits, scales, k, n)
+    bound = _err_bound(x.view(np.float16).astype(np.float32), oracle_mod.dequant_group(codes, bits, scales, n, k))
+    dc, ds, dy = ctx.upload(codes), ctx.upload(scales), ctx.alloc(m * n * 4)
+    dx, dx1 = ctx.upload(x), ctx.upload(np.concatenate([np.zeros(1, x.dtype), x.ravel()]))
+    try:
+        for p in (dx, dx1 + 2):
+            S.qmm(ctx, p, dc, bits, ds, dy, m, n, k)
+            y = ctx.download(dy, (m, n), np.float32)
+            assert np.all(np.abs(y - ref) <= bound), float(np.max(np.abs(y - ref) - bound))
+    finally:
+        for p in (dc, ds, dx, dx1, dy):
+            ctx.free(p)

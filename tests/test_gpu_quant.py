@@ -64,3 +64,30 @@ def test_quantized_model_matches_oracle(gpu_ctx, oracle_mod, bits, n):
     finally:
         kv.close()
         m.close()
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("hidden,inter,n", [(64, 64, 3), (320, 704, 8), (1088, 3136, 2), (2112, 1088, 1)])
+def test_quantized_layer_widths(gpu_ctx, oracle_mod, bits, hidden, inter, n):
+    """The fused quantized projections (RMSNorm, residual and SwiGLU folded in) at widths off their tiles: one scale
+    group, odd numbers of groups, and rows past one and two code loads per wave; a prompt of n <= 8 rows (row kernel),
+    then three decode steps (one-row kernel), against the oracle on the dequantized weights."""
+    cfg = S.QwenConfig(vocab_size=512, hidden_size=hidden, num_hidden_layers=2, num_attention_heads=4,
+                       num_key_value_heads=2, intermediate_size=inter, tie_word_embeddings=False)
+    w = S.synth_weights(cfg, 43, 0.05)
+    m = S.Model(gpu_ctx, cfg).load(w).quantize(bits)
+    om = oracle_mod.OracleModel(cfg, _dequantized(oracle_mod, w, bits))
+    kv = S.KVCache(m, 1, 32)
+    try:
+        ids = S.synth_tokens(44, "widths", cfg.vocab_size, n)
+        lg, tok = S.prefill(m, kv, 0, ids, 0, logit_rows=n)
+        cache = oracle_mod.OracleCache(om, 32)
+        assert_logits_close(lg, cache.forward(ids, 0, logit_rows=n), f"int{bits} {hidden}/{inter}, {n} rows")
+        for i in range(3):
+            lg, t = S.decode(m, kv, 0, tok)
+            r = cache.forward(np.array([tok], np.int32), n + i)
+            assert_logits_close(lg, r[0], f"int{bits} {hidden}/{inter}, decode {i}")
+            tok = t
+    finally:
+        kv.close()
+        m.close()
