@@ -325,16 +325,20 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
     cl[j][t] = ld_dev(pj + HD + 1);
   }
   __syncthreads();
-  if (tid < G) {
+  // a wave per head, a lane per chunk (one thread walking 64 chunks' maxima and exponentials took as long as the
+  // chunk itself)
+  for (int j = wid; j < G; j += 4) {
     float M = -INFINITY;
-    for (int t = 0; t < nact; ++t) M = fmaxf(M, cm[tid][t]);
+    for (int t = lane; t < nact; t += 64) M = fmaxf(M, cm[j][t]);
+    M = wave_max(M);
     float L = 0.0f;
-    for (int t = 0; t < nact; ++t) {
-      const float e = expf(cm[tid][t] - M);
-      cm[tid][t] = e;
-      L += cl[tid][t] * e;
+    for (int t = lane; t < nact; t += 64) {
+      const float e = expf(cm[j][t] - M);
+      cm[j][t] = e;
+      L += cl[j][t] * e;
     }
-    lstat[tid] = L;
+    L = wave_sum(L);
+    if (lane == 0) lstat[j] = L;
   }
   __syncthreads();
 #pragma unroll
