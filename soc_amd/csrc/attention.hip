@@ -27,7 +27,8 @@ constexpr int kMaxCombine = 160;  // key chunks one attention row may be split i
 // alternate chunks to alternate shader engines), so with 8 KV heads XCD g serves head g and every XCD gets the same
 // number of chunks however ragged the rows are. (With the chunk index fastest, rows of few chunks would load only
 // the XCDs and shader engines that low chunk indices map to.)
-template <int G, bool FUSED, int KH>
+// PAIR: outputs as hi/lo pairs (out_hi, out_lo) instead of fp32.
+template <int G, bool FUSED, int KH, bool PAIR>
 __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
   __shared__ float qs[G][HD];
   __shared__ float kn[HD], vn[HD];
@@ -143,6 +144,17 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
   __syncthreads();
 
   const int sub = lane & 15, r = lane >> 4;
+  auto put = [&](int j, int i, float o) {  // one output of query head j
+    const size_t at = static_cast<size_t>(b) * a.ld_out + (g * G + j) * HD + i;
+    if constexpr (PAIR) {
+      __asm__ volatile("" : "+v"(o));  // one fp32 value for both roundings
+      const f16 h = static_cast<f16>(o);
+      a.out_hi[at] = h;
+      a.out_lo[at] = static_cast<f16>((o - static_cast<float>(h)) * 2048.0f);
+    } else {
+      a.out[at] = o;
+    }
+  };
 
   // scores on matrix cores: D[row][key] = Q . K^T with v_mfma_f32_16x16x32_f16 over 16-key tiles, the keys loaded
   // above as B. The A operand rows are the G query heads as fp16 hi = f16(q) and, in rows G..2G-1,
@@ -282,7 +294,7 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
     for (int idx = tid; idx < G * HD; idx += 256) {
       const int j = idx / HD, i = idx % HD;
       const float o = red[0][j][i] + red[1][j][i] + red[2][j][i] + red[3][j][i];
-      a.out[static_cast<size_t>(b) * a.ld_out + (g * G + j) * HD + i] = o / lstat[j];
+      put(j, i, o / lstat[j]);
     }
     return;
   }
@@ -360,7 +372,7 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
       for (int u = 0; u < 16; ++u)
         if (t + u < nact) O += v[u] * ej[t + u];
     }
-    a.out[static_cast<size_t>(b) * a.ld_out + (g * G + j) * HD + i] = O / lstat[j];
+    put(j, i, O / lstat[j]);
   }
   if (tid == 0) st_dev(a.counters + b * a.nkv + g, 0);
 }
@@ -1090,14 +1102,16 @@ hipError_t launch_attention(const AttnArgs& a, int fused, hipStream_t s) {
   const int G = a.nq / a.nkv;
   if (a.chunk > 256 || a.chunk <= 0) return hipErrorInvalidValue;
   if (a.max_split > kMaxCombine) return hipErrorInvalidValue;
+  if (a.out_hi != nullptr ? a.out_lo == nullptr || fused : a.out == nullptr) return hipErrorInvalidValue;
   const dim3 grid(a.nkv, a.max_split, a.B), block(256);
   // unfused rows (the ragged batch): keys and values in halves, 88 instead of 112 registers, five blocks per CU
   // instead of four (Qwen3-4B x 16 ragged step 4.07 -> 4.04 ms); the fused single-sequence decode runs few blocks and
   // keeps the one round trip per operand
 #define SOC_ATTN_CASE(GG)                                                                  \
   if (G == GG) {                                                                          \
-    if (fused) hipLaunchKernelGGL((k_attention<GG, true, 1>), grid, block, 0, s, a);       \
-    else hipLaunchKernelGGL((k_attention<GG, false, 2>), grid, block, 0, s, a);            \
+    if (fused) hipLaunchKernelGGL((k_attention<GG, true, 1, false>), grid, block, 0, s, a);             \
+    else if (a.out_hi != nullptr) hipLaunchKernelGGL((k_attention<GG, false, 2, true>), grid, block, 0, s, a); \
+    else hipLaunchKernelGGL((k_attention<GG, false, 2, false>), grid, block, 0, s, a);                  \
     return hipGetLastError();                                                             \
   }
   SOC_ATTN_CASE(1)

@@ -8,7 +8,7 @@
 
 namespace soc {
 
-enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_QKV = 3 };
+enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_QKV = 3, EPI_PART = 4 };
 
 // ---- decode GEMV (batch 1) ----
 struct GemvArgs {
@@ -89,7 +89,8 @@ struct AttnArgs {
   int pos_base;          // added to pos[] (prefill rows use pos = nullptr and pos_base + row)
   float* out;            // [B][nq*d] (prefill MFMA kernel: may be null when out_hi / out_lo are set)
   int ld_out;
-  f16* out_hi;           // prefill MFMA kernel: optional hi = f16(o), lo = f16((o - hi) * 2^11) copies [B][ld_out]
+  f16* out_hi;           // optional hi = f16(o), lo = f16((o - hi) * 2^11) copies [B][ld_out]; the row kernel
+                         // (launch_attention) then writes both and leaves out alone
   f16* out_lo;
   float* part;           // split partials [B][nq][max_split][d + 2]
   int* counters;         // [B][nkv] zero-initialised
@@ -287,9 +288,23 @@ struct GemmSplitArgs {
     int slot, layer, cap, pos_base, nq, nkv;
     float eps;
   } qkv;
+  int splits;  // set by launch_gemm_rows
 };
 bool gemm_split_supported(const GemmSplitArgs& g);
 hipError_t launch_gemm_split(const GemmSplitArgs& g, int epi, hipStream_t s);
+
+// Projection of a ragged decode batch of any number of rows, K % 32 == 0, hi/lo activations: the split-K partial sums
+// c [splits][M][N] (splits = gemm_rows_splits(M, N, K); gemm_rows_part_floats(M, N) floats suffice). w2: the second half
+// of the N rows (gate | up). launch_rows_*: the sums added in split order and what follows in the layer (rows_epi.hip):
+// x += sums and RMSNorm(x) as a hi/lo pair; silu(gate) * up as a hi/lo pair; the attention input (a.T rows, a.pos and
+// a.slots set, a.qkv unused).
+int gemm_rows_splits(int M, int N, int K);
+size_t gemm_rows_part_floats(int M, int N);
+hipError_t launch_gemm_rows(const GemmSplitArgs& g, hipStream_t s);
+hipError_t launch_rows_residual_norm(const float* part, int splits, int M, int H, float* x, const f16* gain, float eps,
+                                     f16* yh, f16* yl, hipStream_t s);
+hipError_t launch_rows_swiglu(const float* part, int splits, int M, int I, f16* yh, f16* yl, hipStream_t s);
+hipError_t launch_rows_qkv(const float* part, int splits, const QkNormRopeArgs& a, hipStream_t s);
 
 // Skinny projection of a ragged decode batch: x[M][K] . [w | w2]^T for 1 <= M <= 16 rows, K % 256 == 0, split over
 // K, then an epilogue kernel that adds the splits in order. Rows 0..N0-1 come from w, rows N0..Ntot-1 from w2.

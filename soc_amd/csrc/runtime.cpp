@@ -119,6 +119,7 @@ struct BatchWs {
   // per-row candidates and arrival counters of the split greedy argmax ([cap][kArgmaxMaxChunks], [cap])
   float* am_val = nullptr;
   int32_t *am_idx = nullptr, *am_cnt = nullptr;
+  float* part = nullptr;  // split-K partial sums of the row GEMMs
   std::vector<void*> allocs;
   int32_t* ring = nullptr;  // [rows][steps] tokens of soc_decode_batch_steps
   size_t ring_cap = 0;
@@ -897,25 +898,6 @@ hipError_t split_gemm(const soc::f16* ah, const soc::f16* al, int lda, const soc
   return soc::launch_gemm_split(g, epi, s);
 }
 
-// A ragged-batch projection on the skinny kernel, in chunks of 16 rows: `proto` carries the weights, the input
-// RMSNorm gain (or none) and the epilogue's own arguments; rows m0.. of x, c, q_out, pos and slots per chunk.
-hipError_t batch_skinny(const soc::SkinnyArgs& proto, int n, int epi, hipStream_t s) {
-  for (int m0 = 0; m0 < n; m0 += 16) {
-    soc::SkinnyArgs a = proto;
-    a.x = proto.x + static_cast<size_t>(m0) * proto.ldx;
-    a.M = std::min(16, n - m0);
-    if (proto.c != nullptr) a.c = proto.c + static_cast<size_t>(m0) * proto.ldc;
-    if (epi == soc::EPI_QKV) {
-      a.q_out = proto.q_out + static_cast<size_t>(m0) * proto.nq * 128;
-      a.pos = proto.pos + m0;
-      a.slots = proto.slots + m0;
-    }
-    const hipError_t e = soc::launch_skinny(a, epi, s);
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
-}
-
 // Largest split-K scratch any projection of the model needs in the skinny kernel (floats).
 size_t skinny_scratch_floats(const soc_model* m) {
   const soc_qwen_config& c = m->cfg;
@@ -958,9 +940,16 @@ int validate_ids(const soc_model* m, const int32_t* ids, int n) {
 }
 
 
+// A batch step's projections: the skinny kernels (input RMSNorm, q/k norm, RoPE and KV append folded in) up to their 16
+// rows, else the split-K row GEMMs, which stream the weights once whatever the rows (two layers and a 16384-word head,
+// us per step, against skinny slabs of 16: Qwen3-0.6B 17 rows 198 : 277, 64 rows 226 : 470; Qwen3-4B 17 rows 329 : 400,
+// 64 rows 374 : 703).
+bool batch_skinny_path(const soc_model* m, int n) { return m->pws.skpart != nullptr && n <= 16; }
+
 int ensure_batch_ws(soc_model* m, int n) {
   BatchWs& b = m->bws;
-  if (b.cap >= n) return SOC_OK;
+  const bool rows = !batch_skinny_path(m, n);  // needs the row GEMMs' partial sums
+  if (b.cap >= n && (b.part != nullptr || !rows)) return SOC_OK;
   hipError_t e = hipStreamSynchronize(m->ctx->stream);
   if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
   free_all(b.allocs);
@@ -977,6 +966,8 @@ int ensure_batch_ws(soc_model* m, int n) {
   SOC_TRY(dev_alloc_t(b.allocs, n, &b.am_cnt));
   if ((e = hipMemset(b.am_cnt, 0, static_cast<size_t>(n) * sizeof(int32_t))) != hipSuccess)
     return hip_fail(e, "hipMemset");
+  const int columns = std::max({m->qkv_rows, 2 * m->cfg.intermediate_size, m->cfg.hidden_size});
+  if (rows) SOC_TRY(dev_alloc_t(b.allocs, soc::gemm_rows_part_floats(n, columns), &b.part));
   b.cap = n;
   return SOC_OK;
 }
@@ -1015,16 +1006,30 @@ int enqueue_batch_step(soc_model* m, soc_kv* kv, int n, int max_split, int32_t* 
   hipStream_t s = m->ctx->stream;
   const int H = c.hidden_size, I = c.intermediate_size;
   hipError_t e;
-  // up to 64 rows: the skinny kernels per projection and 16 rows (input RMSNorm and the q/k norm, RoPE and KV append
-  // folded into them); beyond, the tile GEMMs with separate normalisation and q/k kernels
-  const bool fused = w.skpart != nullptr && n <= 64;
-  soc::SkinnyArgs sk{};
-  sk.part = w.skpart;
-  sk.eps = c.rms_norm_eps;
   if ((e = soc::launch_embed(b.ids, n, m->embed, H, w.x, s)) != hipSuccess) return hip_fail(e, "embed");
-  for (int l = 0; l < c.num_hidden_layers; ++l) {
-    const DevLayer& L = m->layers[l];
-    if (fused) {
+  auto attention = [&](int l, f16* hi, f16* lo) -> hipError_t {
+    soc::AttnArgs at = attn_args(m, kv, l);
+    at.qkv = w.q;
+    at.ld_qkv = m->qd;
+    at.pos = b.pos;
+    at.slot = b.slots;
+    at.out = w.attn;
+    at.out_hi = hi;
+    at.out_lo = lo;
+    at.ld_out = m->qd;
+    at.part = w.part;
+    at.counters = w.attn_counters;
+    at.B = n;
+    at.max_split = max_split;
+    return soc::launch_attention(at, 0, s);
+  };
+  if (batch_skinny_path(m, n)) {
+    soc::SkinnyArgs sk{};
+    sk.M = n;
+    sk.part = w.skpart;
+    sk.eps = c.rms_norm_eps;
+    for (int l = 0; l < c.num_hidden_layers; ++l) {
+      const DevLayer& L = m->layers[l];
       soc::SkinnyArgs a = sk;
       a.x = w.x;
       a.ldx = H;
@@ -1047,24 +1052,73 @@ int enqueue_batch_step(soc_model* m, soc_kv* kv, int n, int max_split, int32_t* 
       a.cap = kv->cap;
       a.nq = c.num_attention_heads;
       a.nkv = c.num_key_value_heads;
-      if ((e = batch_skinny(a, n, soc::EPI_QKV, s)) != hipSuccess) return hip_fail(e, "skinny qkv");
-    } else {
-      if ((e = soc::launch_rmsnorm_rows(w.x, n, H, L.in_norm, c.rms_norm_eps, w.xn, nullptr, nullptr, s)) !=
-          hipSuccess)
-        return hip_fail(e, "rmsnorm");
-      soc::GemmArgs g{};
-      g.a = w.xn;
-      g.lda = H;
-      g.w = L.wqkv;
-      g.c = w.qkv;
-      g.ldc = m->qkv_rows;
+      if ((e = soc::launch_skinny(a, soc::EPI_QKV, s)) != hipSuccess) return hip_fail(e, "skinny qkv");
+      if ((e = attention(l, nullptr, nullptr)) != hipSuccess) return hip_fail(e, "attention");
+      a = sk;  // o: x += attn . Wo^T
+      a.x = w.attn;
+      a.ldx = m->qd;
+      a.w = L.wo;
+      a.N0 = a.Ntot = H;
+      a.K = m->qd;
+      a.c = w.x;
+      a.ldc = H;
+      if ((e = soc::launch_skinny(a, soc::EPI_RESIDUAL, s)) != hipSuccess) return hip_fail(e, "skinny o");
+      a = sk;  // gate/up of RMSNorm(x) + SwiGLU
+      a.x = w.x;
+      a.ldx = H;
+      a.w = L.wgate;
+      a.w2 = L.wup;
+      a.N0 = I;
+      a.Ntot = 2 * I;
+      a.K = H;
+      a.gain = L.post_norm;
+      a.c = w.h;
+      a.ldc = I;
+      if ((e = soc::launch_skinny(a, soc::EPI_SWIGLU, s)) != hipSuccess) return hip_fail(e, "skinny gate/up");
+      a = sk;  // down: x += h . Wd^T
+      a.x = w.h;
+      a.ldx = I;
+      a.w = L.wdown;
+      a.N0 = a.Ntot = H;
+      a.K = I;
+      a.c = w.x;
+      a.ldc = H;
+      if ((e = soc::launch_skinny(a, soc::EPI_RESIDUAL, s)) != hipSuccess) return hip_fail(e, "skinny down");
+    }
+    soc::SkinnyArgs a = sk;  // LM head of RMSNorm(x) with the final gain
+    a.x = w.x;
+    a.ldx = H;
+    a.w = m->lm_head;
+    a.N0 = a.Ntot = c.vocab_size;
+    a.K = H;
+    a.gain = m->final_norm;
+    a.c = w.logits;
+    a.ldc = c.vocab_size;
+    if ((e = soc::launch_skinny(a, soc::EPI_STORE, s)) != hipSuccess) return hip_fail(e, "skinny lm head");
+  } else {
+    // hi/lo activation pairs throughout; each projection's split sums are finished by the kernel that makes the next
+    // one's input
+    auto rows = [&](const f16* ah, const f16* al, const f16* wt, const f16* w2, int N, int K) -> hipError_t {
+      soc::GemmSplitArgs g{};
+      g.ah = ah;
+      g.al = al;
+      g.lda = K;
+      g.w = wt;
+      g.w2 = w2;
+      g.c = b.part;
+      g.ldc = N;
       g.M = n;
-      g.N = m->qkv_rows;
-      g.K = H;
-      if ((e = prefill_gemm(g, soc::EPI_STORE, s)) != hipSuccess) return hip_fail(e, "gemm qkv");
+      g.N = N;
+      g.K = K;
+      return soc::launch_gemm_rows(g, s);
+    };
+    if ((e = soc::launch_rmsnorm_rows(w.x, n, H, m->layers[0].in_norm, c.rms_norm_eps, nullptr, w.ph, w.pl, s)) !=
+        hipSuccess)
+      return hip_fail(e, "rmsnorm");
+    for (int l = 0; l < c.num_hidden_layers; ++l) {
+      const DevLayer& L = m->layers[l];
+      if ((e = rows(w.ph, w.pl, L.wqkv, nullptr, m->qkv_rows, H)) != hipSuccess) return hip_fail(e, "rows qkv");
       soc::QkNormRopeArgs q{};
-      q.qkv = w.qkv;
-      q.ld_qkv = m->qkv_rows;
       q.q_gain = L.q_norm;
       q.k_gain = L.k_norm;
       q.eps = c.rms_norm_eps;
@@ -1082,112 +1136,25 @@ int enqueue_batch_step(soc_model* m, soc_kv* kv, int n, int max_split, int32_t* 
       q.nkv = c.num_key_value_heads;
       q.pos = b.pos;
       q.slots = b.slots;
-      if ((e = soc::launch_qk_norm_rope_append(q, s)) != hipSuccess) return hip_fail(e, "qk norm rope");
+      if ((e = soc::launch_rows_qkv(b.part, soc::gemm_rows_splits(n, m->qkv_rows, H), q, s)) != hipSuccess)
+        return hip_fail(e, "rows q/k norm");
+      if ((e = attention(l, w.ph, w.pl)) != hipSuccess) return hip_fail(e, "attention");
+      if ((e = rows(w.ph, w.pl, L.wo, nullptr, H, m->qd)) != hipSuccess) return hip_fail(e, "rows o");
+      if ((e = soc::launch_rows_residual_norm(b.part, soc::gemm_rows_splits(n, H, m->qd), n, H, w.x, L.post_norm,
+                                              c.rms_norm_eps, w.ph, w.pl, s)) != hipSuccess)
+        return hip_fail(e, "rows residual");
+      if ((e = rows(w.ph, w.pl, L.wgate, L.wup, 2 * I, H)) != hipSuccess) return hip_fail(e, "rows gate/up");
+      if ((e = soc::launch_rows_swiglu(b.part, soc::gemm_rows_splits(n, 2 * I, H), n, I, w.qh, w.ql, s)) != hipSuccess)
+        return hip_fail(e, "rows swiglu");
+      if ((e = rows(w.qh, w.ql, L.wdown, nullptr, H, I)) != hipSuccess) return hip_fail(e, "rows down");
+      const f16* next = l + 1 < c.num_hidden_layers ? m->layers[l + 1].in_norm : m->final_norm;
+      if ((e = soc::launch_rows_residual_norm(b.part, soc::gemm_rows_splits(n, H, I), n, H, w.x, next, c.rms_norm_eps,
+                                              w.ph, w.pl, s)) != hipSuccess)
+        return hip_fail(e, "rows residual");
     }
-    soc::AttnArgs at = attn_args(m, kv, l);
-    at.qkv = w.q;
-    at.ld_qkv = m->qd;
-    at.pos = b.pos;
-    at.slot = b.slots;
-    at.out = w.attn;
-    at.ld_out = m->qd;
-    at.part = w.part;
-    at.counters = w.attn_counters;
-    at.B = n;
-    at.max_split = max_split;
-    if ((e = soc::launch_attention(at, 0, s)) != hipSuccess) return hip_fail(e, "attention");
-    if (fused) {
-      soc::SkinnyArgs a = sk;  // o: x += attn . Wo^T
-      a.x = w.attn;
-      a.ldx = m->qd;
-      a.w = L.wo;
-      a.N0 = a.Ntot = H;
-      a.K = m->qd;
-      a.c = w.x;
-      a.ldc = H;
-      if ((e = batch_skinny(a, n, soc::EPI_RESIDUAL, s)) != hipSuccess) return hip_fail(e, "skinny o");
-      a = sk;  // gate/up of RMSNorm(x) + SwiGLU
-      a.x = w.x;
-      a.ldx = H;
-      a.w = L.wgate;
-      a.w2 = L.wup;
-      a.N0 = I;
-      a.Ntot = 2 * I;
-      a.K = H;
-      a.gain = L.post_norm;
-      a.c = w.h;
-      a.ldc = I;
-      if ((e = batch_skinny(a, n, soc::EPI_SWIGLU, s)) != hipSuccess) return hip_fail(e, "skinny gate/up");
-      a = sk;  // down: x += h . Wd^T
-      a.x = w.h;
-      a.ldx = I;
-      a.w = L.wdown;
-      a.N0 = a.Ntot = H;
-      a.K = I;
-      a.c = w.x;
-      a.ldc = H;
-      if ((e = batch_skinny(a, n, soc::EPI_RESIDUAL, s)) != hipSuccess) return hip_fail(e, "skinny down");
-      continue;
-    }
-    soc::GemmArgs g{};
-    g.a = w.attn;
-    g.lda = m->qd;
-    g.w = L.wo;
-    g.c = w.x;
-    g.ldc = H;
-    g.M = n;
-    g.N = H;
-    g.K = m->qd;
-    if ((e = prefill_gemm(g, soc::EPI_RESIDUAL, s)) != hipSuccess) return hip_fail(e, "gemm o");
-    if ((e = soc::launch_rmsnorm_rows(w.x, n, H, L.post_norm, c.rms_norm_eps, w.xn, nullptr, nullptr, s)) != hipSuccess)
-      return hip_fail(e, "rmsnorm");
-    g = soc::GemmArgs{};
-    g.a = w.xn;
-    g.lda = H;
-    g.w = L.wgate;
-    g.w2 = L.wup;
-    g.c = w.h;
-    g.ldc = I;
-    g.M = n;
-    g.N = I;
-    g.K = H;
-    if ((e = prefill_gemm(g, soc::EPI_SWIGLU, s)) != hipSuccess) return hip_fail(e, "gemm gate/up");
-    g = soc::GemmArgs{};
-    g.a = w.h;
-    g.lda = I;
-    g.w = L.wdown;
-    g.c = w.x;
-    g.ldc = H;
-    g.M = n;
-    g.N = H;
-    g.K = I;
-    if ((e = prefill_gemm(g, soc::EPI_RESIDUAL, s)) != hipSuccess) return hip_fail(e, "gemm down");
-  }
-  if (fused) {
-    soc::SkinnyArgs a = sk;  // LM head of RMSNorm(x) with the final gain
-    a.x = w.x;
-    a.ldx = H;
-    a.w = m->lm_head;
-    a.N0 = a.Ntot = c.vocab_size;
-    a.K = H;
-    a.gain = m->final_norm;
-    a.c = w.logits;
-    a.ldc = c.vocab_size;
-    if ((e = batch_skinny(a, n, soc::EPI_STORE, s)) != hipSuccess) return hip_fail(e, "skinny lm head");
-  } else {
-    if ((e = soc::launch_rmsnorm_rows(w.x, n, H, m->final_norm, c.rms_norm_eps, w.xn, nullptr, nullptr, s)) !=
-        hipSuccess)
-      return hip_fail(e, "rmsnorm");
-    soc::GemmArgs g{};
-    g.a = w.xn;
-    g.lda = H;
-    g.w = m->lm_head;
-    g.c = w.logits;
-    g.ldc = c.vocab_size;
-    g.M = n;
-    g.N = c.vocab_size;
-    g.K = H;
-    if ((e = prefill_gemm(g, soc::EPI_STORE, s)) != hipSuccess) return hip_fail(e, "gemm lm head");
+    if ((e = split_gemm(w.ph, w.pl, H, m->lm_head, nullptr, w.logits, nullptr, nullptr, c.vocab_size, n, c.vocab_size, H,
+                        soc::EPI_STORE, s)) != hipSuccess)
+      return hip_fail(e, "gemm lm head");
   }
   if ((e = soc::launch_argmax_rows(w.logits, c.vocab_size, n, b.ids, b.pos, b.start, ring, ring_stride, b.am_val,
                                    b.am_idx, b.am_cnt, s)) != hipSuccess)

@@ -250,3 +250,45 @@ def test_batch_error_paths(gpu_ctx):
     finally:
         kv.close()
         m.close()
+
+
+@pytest.mark.parametrize("n", [17, 64, 65, 128, 130])
+def test_batch_row_gemm_edges(gpu_ctx, n):
+    """The split-K row GEMMs of more than 16 rows at the edges of their 64- and 128-row tiles, widths off the 128-column
+    tiles (hidden 352, intermediate 480): rows agree with single-sequence decode within the model tolerance, permuting
+    them permutes the results bit for bit, and the captured steps equal the eager ones."""
+    cfg = S.QwenConfig(vocab_size=1000, hidden_size=352, num_hidden_layers=2, num_attention_heads=4,
+                       num_key_value_heads=2, intermediate_size=480, tie_word_embeddings=False)
+    m = S.Model(gpu_ctx, cfg).load(S.synth_weights(cfg, 51))
+    kvs = [S.KVCache(m, n, 300) for _ in range(2)]
+    try:
+        last = np.zeros(n, np.int32)
+        for kv in kvs:
+            for slot in range(n):
+                plen = 270 if slot == 3 else 1 + slot % 5  # one row over two attention chunks
+                _, last[slot] = S.prefill(m, kv, slot, S.synth_tokens(60 + slot, "rows", cfg.vocab_size, plen), 0,
+                                          logit_rows=0)
+        order = np.random.RandomState(n).permutation(n).astype(np.int32)
+        lg, nxt = S.decode_batch(m, kvs[0], order, last[order])
+        ident = np.arange(n, dtype=np.int32)
+        lg2, nxt2 = S.decode_batch(m, kvs[1], ident, last)
+        assert np.array_equal(lg2[order], lg) and np.array_equal(nxt2[order], nxt)
+        for kv in kvs:
+            for slot in range(n):
+                kv_len = 270 if slot == 3 else 1 + slot % 5
+                S.capi.check(S.lib().soc_kv_set_length(kv.h, slot, kv_len))
+        for slot in (0, 3, n - 1):
+            ref, t = S.decode(m, kvs[1], slot, int(last[slot]))
+            assert_logits_close(lg2[slot], ref, f"{n} rows, slot {slot}")
+            assert int(nxt2[slot]) == t
+            S.capi.check(S.lib().soc_kv_set_length(kvs[1].h, slot, 270 if slot == 3 else 1 + slot % 5))
+        steps = S.decode_batch_steps(m, kvs[0], ident, last, 3)
+        tok, loop = last.copy(), []
+        for _ in range(3):
+            _, tok = S.decode_batch(m, kvs[1], ident, tok)
+            loop.append(tok.copy())
+        assert np.array_equal(steps, np.stack(loop))
+    finally:
+        for kv in kvs:
+            kv.close()
+        m.close()
