@@ -185,8 +185,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(GemmArgs g) {
 // own loads of slice kt + 1 (vmcnt) and for its LDS reads (lgkmcnt). The MFMA operands of the next 16-deep step are
 // read from LDS while the current step's MFMAs run (two register sets used in turn), one read issued after each
 // MFMA. Rows are BK halves with the 16-byte chunk c of row r stored at slot c ^ ((r >> 2) & 3) (BK = 32) or
-// c ^ ((r >> 1) & 7) (BK = 64): the 16 rows a b128 read phase touches land on different bank groups.
-// BM x BN tile per block of NWM x NWN waves (each a (BM/NWM) x (BN/NWN) part, v_mfma_f32_32x32x16_f16; every
+// c ^ ((r >> 1) & 7) (BK = 64) or c ^ (r & 15) (BK = 128): the 16 rows a b128 read phase touches land on different bank groups.
+// BM x BN tile per block of NWM x NWN waves (each a (BM/NWM) x (BN/NWN) part, v_mfma_f32_32x32x16_f16), NLD waves
+// loading (those beyond NWM x NWN do nothing else: a small tile has more loads than its waves can keep in flight; every
 // configuration accumulates the same 16-deep MFMA steps in the same K order). Tiles are dealt to the
 // eight XCDs as an mx x (8 / mx) grid of rectangles (block b runs on XCD b % 8), mx chosen to minimise the bytes
 // of A and W each XCD's L2 has to fetch. The products and their order match k_gemm_mfma<EPI, true, .> exactly, or
@@ -197,11 +198,12 @@ namespace {
 // LDS has 64 banks of 4 bytes, and a 16-byte read serves 16 lanes per cycle: the 16 rows one read phase touches
 // (lanes 0-15, 16-31, ...) must hit 16 different 16-byte bank groups. A 64-half row is half a bank row, so rows r and
 // r + 1 sit in different halves and the slot must differ between rows of equal parity: c ^ ((r >> 1) & 7). A
-// 32-half row is a quarter: c ^ ((r >> 2) & 3).
+// 32-half row is a quarter: c ^ ((r >> 2) & 3). A 128-half row is a whole one: c ^ (r & 15).
 template <int BK>
 __device__ __forceinline__ int chunk_slot(int r, int c) {
   if constexpr (BK == 32) return c ^ ((r >> 2) & 3);
-  else return c ^ ((r >> 1) & 7);
+  else if constexpr (BK == 64) return c ^ ((r >> 1) & 7);
+  else return c ^ (r & 15);
 }
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
@@ -229,21 +231,22 @@ __device__ __forceinline__ void block_barrier() {
 }
 }  // namespace
 
-template <int EPI, int BM, int BN, int ST, int MINB, int BK, bool LO, int NWM, int NWN>
-__global__ __launch_bounds__(64 * NWM * NWN, MINB) void k_gemm_split(GemmSplitArgs g, int mx) {
+template <int EPI, int BM, int BN, int ST, int MINB, int BK, bool LO, int NWM, int NWN, int NLD>
+__global__ __launch_bounds__(64 * NLD, MINB) void k_gemm_split(GemmSplitArgs g, int mx) {
   constexpr int NW = NWM * NWN;                    // waves: NWM x NWN, each a WTM x WTN part of the tile
   constexpr int WTM = BM / NWM, WTN = BN / NWN;
   constexpr int MI = WTM / 32, NJ = WTN / 32;      // 32x32 MFMA tiles per wave
   constexpr int RPI = 1024 / (BK * 2);             // rows per 1 KB wave instruction
   constexpr int CPR = BK / 8;                      // 16-byte chunks per row
   constexpr int AP = LO ? 2 : 1;                   // activation parts: hi and lo, or hi alone
-  constexpr int AI = BM / RPI / NW, WI = BN / RPI / NW;  // DMA instructions per wave per slice: each A part, W
+  constexpr int AI = BM / RPI / NLD, WI = BN / RPI / NLD;  // DMA instructions per wave per slice: each A part, W
   constexpr int IPT = AP * AI + WI;
   constexpr int KS = BK / 16;  // 16-deep MFMA steps per slice
   constexpr int STAGE_H = (AP * BM + BN) * BK;
   static_assert(EPI != EPI_SWIGLU || NJ % 2 == 0, "SwiGLU pairs gate and up tiles within a wave");
   static_assert(KS % 2 == 0 && ST >= 2 && AI >= 1 && WI >= 1, "tile shape");
-  static_assert(AI * RPI * NW == BM && WI * RPI * NW == BN && MI >= 1 && NJ >= 1, "tile shape");
+  static_assert(AI * RPI * NLD == BM && WI * RPI * NLD == BN && MI >= 1 && NJ >= 1, "tile shape");
+  static_assert(NLD == NW || (NLD > NW && EPI != EPI_QKV), "loader waves");
   extern __shared__ __attribute__((aligned(16))) _Float16 slds[];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int wm = wid / NWN, wn = wid % NWN;
@@ -368,6 +371,14 @@ __global__ __launch_bounds__(64 * NWM * NWN, MINB) void k_gemm_split(GemmSplitAr
     if (p < KT) issue(p, p);
   wait_slices<IPT, ST - 1>(KT - 1);
   block_barrier();
+  if (NLD > NW && wid >= NW) {  // loader waves: the slices' waits, barriers and refills alone
+    for (int kt = 0; kt + 1 < KT; ++kt) {
+      wait_slices<IPT, ST - 2>(KT - 2 - kt);
+      block_barrier();
+      if (kt + ST < KT) issue(kt + ST, kt % ST);
+    }
+    return;
+  }
   read(a0, b0, 0, 0);
   for (int kt = 0; kt < KT; ++kt) {
     const int st = kt % ST;
@@ -548,7 +559,7 @@ int xcd_split(int mt, int nt, double abytes, double wbytes) {
   return best;
 }
 
-template <int EPI, int BM, int BN, int ST, int MINB, int BK, bool LO, int NWM = 2, int NWN = 2>
+template <int EPI, int BM, int BN, int ST, int MINB, int BK, bool LO, int NWM = 2, int NWN = 2, int NLD = NWM * NWN>
 hipError_t launch_split_cfg(const GemmSplitArgs& g, hipStream_t s) {
   constexpr int AP = LO ? 2 : 1;
   const int bn = EPI == EPI_SWIGLU ? BN / 2 : BN;
@@ -559,50 +570,83 @@ hipError_t launch_split_cfg(const GemmSplitArgs& g, hipStream_t s) {
   const int splits = EPI == EPI_PART ? g.splits : 1;
   const size_t lds = static_cast<size_t>(ST) * (AP * BM + BN) * BK * sizeof(_Float16);
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(k_gemm_split<EPI, BM, BN, ST, MINB, BK, LO, NWM, NWN>),
+      reinterpret_cast<const void*>(k_gemm_split<EPI, BM, BN, ST, MINB, BK, LO, NWM, NWN, NLD>),
       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((k_gemm_split<EPI, BM, BN, ST, MINB, BK, LO, NWM, NWN>), dim3(mt * nt * splits), dim3(64 * NWM * NWN),
+  hipLaunchKernelGGL((k_gemm_split<EPI, BM, BN, ST, MINB, BK, LO, NWM, NWN, NLD>), dim3(mt * nt * splits), dim3(64 * NLD),
                      lds, s,
                      g, mx);
   return hipGetLastError();
 }
 
+// The tile of a projection by how many blocks it makes of M and N. A block's K loop waits on its loads far more than on
+// its MFMAs unless the chip is full of large tiles, so the tile shrinks until about every CU has a block (a block's time
+// then falls with its bytes per K), and a small tile takes the LDS left over for a deep ring of 128-deep slices (at
+// most 160 KB; slices of 128 halve the barriers; four waves load for one or two that compute). Every tile accumulates
+// the same 16-deep MFMA steps in the same K order: bit-identical rows whatever the tile.
 template <int EPI>
 hipError_t launch_split_epi(const GemmSplitArgs& g, hipStream_t s) {
-  // 128-row tiles on 8 waves when they still give every CU its blocks (long prompts; measured on the Qwen3-0.6B
-  // prefill at 2048 tokens): a block's 8 waves share twice the rows of A and W per LDS slice, and two such blocks per
-  // CU keep 16 waves resident. QKV (hi/lo activations): 128 x 128 tiles, 32-deep slices in a 3-slot ring (56 -> 53
-  // us); gate/up: 128 x 128 (64 gate and 64 up rows), 64-deep slices in a 2-slot ring (44 -> 39.5 us); o/down
-  // (N <= 1024, one block per CU): 128 x 64, a 4-slot ring (29 -> 28 us).
-  const int mt128 = (g.M + 127) / 128;
+  const bool deep = g.K % 128 == 0;
+  auto blocks = [&](int bm, int bn) { return ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
+  // rounds of the whole chip at `slots` blocks a round
+  auto rounds = [](int b, int slots) { return (b + slots - 1) / slots; };
   if constexpr (EPI == EPI_QKV) {
-    if (g.al != nullptr && mt128 * (g.N / 128) >= 512) return launch_split_cfg<EPI, 128, 128, 3, 2, 32, true, 4, 2>(g, s);
-  }
-  if constexpr (EPI == EPI_STORE) {  // the batch's LM head: the same tile
-    if (g.al != nullptr && g.M > 64 && mt128 * ((g.N + 127) / 128) >= 512)
+    // Tiles of one 128-column head. Per layer against 64 x 128 tiles two a CU, us: 32 rows, Qwen3-0.6B 31 tokens -4.8,
+    // 200 -4.1, Qwen3-4B 31 -18.0, 128 -18.6; 64 rows on 8 waves, Qwen3-0.6B 333 -2.8, Qwen3-1.7B 333 -9.6. Large:
+    // 128 x 128 (8 waves, 32-deep slices in a 3-slot ring, two a CU) where it halves the rounds of 512 blocks
+    // (Qwen3-0.6B 2048 tokens, one against two: -4.9); Qwen3-4B 1500, two against three, is 7.4 slower with it.
+    if (g.al != nullptr && deep && blocks(32, 128) <= 256) return launch_split_cfg<EPI, 32, 128, 3, 1, 128, true, 1, 4>(g, s);
+    if (g.al != nullptr && g.K % 64 == 0 && blocks(64, 128) <= 256)
+      return launch_split_cfg<EPI, 64, 128, 4, 1, 64, true, 2, 4>(g, s);
+    const int b = blocks(128, 128);
+    if (g.al != nullptr && b >= 512 && 2 * rounds(b, 512) <= rounds(blocks(64, 128), 512))
       return launch_split_cfg<EPI, 128, 128, 3, 2, 32, true, 4, 2>(g, s);
   }
   if constexpr (EPI == EPI_SWIGLU) {
-    // gate/up of a full chip of 256-row tiles: 256 x 192 (96 gate and 96 up rows) on 8 waves of 32 rows, one block
-    // per CU, one tile each (2048 tokens: 39.7 -> 37.9 us; 128 x 128 tiles make 1.5 rounds of two blocks per CU)
-    if (g.al == nullptr && g.K % 64 == 0 && ((g.M + 255) / 256) * ((g.N + 95) / 96) >= 256)
-      return launch_split_cfg<EPI, 256, 192, 2, 1, 64, false, 8, 1>(g, s);
-    if (g.al == nullptr && g.K % 64 == 0 && mt128 * ((g.N + 63) / 64) >= 512)
-      return launch_split_cfg<EPI, 128, 128, 2, 2, 64, false, 4, 2>(g, s);
+    // BN / 2 outputs (gate and up rows) per tile. Per layer against 64 x 128, us: 32 x 64 Qwen3-0.6B 64 rows -4.0,
+    // Qwen3-1.7B 31 -15.9; 32 x 128 Qwen3-4B 31 -13.7; 64 x 64 Qwen3-0.6B 100 -3.1; 64 x 128 in three 128-deep slots
+    // Qwen3-4B 64 -10.0; 128 x 128 in four slots Qwen3-8B 100 -13.6, Qwen3-0.6B 333 +0.3.
+    if (g.al == nullptr && deep) {
+      if (blocks(32, 32) <= 256) return launch_split_cfg<EPI, 32, 64, 3, 2, 128, false, 1, 1, 4>(g, s);
+      if (g.M <= 32 && blocks(32, 64) <= 256) return launch_split_cfg<EPI, 32, 128, 3, 1, 128, false, 1, 2, 4>(g, s);
+      if (blocks(64, 32) <= 256) return launch_split_cfg<EPI, 64, 64, 2, 2, 128, false, 2, 1, 4>(g, s);
+      if (blocks(64, 64) <= 256) return launch_split_cfg<EPI, 64, 128, 3, 1, 128, false, 2, 2>(g, s);
+      if (blocks(128, 64) <= 256) return launch_split_cfg<EPI, 128, 128, 4, 1, 64, false, 4, 2>(g, s);
+    }
+    // Large: the cheapest of 256 x 192 (96 gate and 96 up rows, 8 waves, one a CU), 128 x 128 and 64 x 128 (two a CU)
+    // by rounds times a round's time, which goes with its outputs (24576, 16384 and 8192 a CU, the smaller tiles a
+    // little dearer per output). 256 x 192 against 128 x 128, us per layer: Qwen3-8B 2000 tokens -54 (4 rounds to 6),
+    // Qwen3-4B 512 -16 (1 to 2), 700 +28 (2 to 2), 1500 +16 (3 to 4), 2048 +17 (4 to 5).
+    if (g.al == nullptr && g.K % 64 == 0) {
+      const double c256 = 1.5 * rounds(blocks(256, 96), 256), c128 = 1.12 * rounds(blocks(128, 64), 512),
+                   c64 = 0.64 * rounds(blocks(64, 64), 512);
+      if (c256 <= c128 && c256 <= c64) return launch_split_cfg<EPI, 256, 192, 2, 1, 64, false, 8, 1>(g, s);
+      if (c128 <= c64) return launch_split_cfg<EPI, 128, 128, 2, 2, 64, false, 4, 2>(g, s);
+    }
+  }
+  if constexpr (EPI == EPI_RESIDUAL) {
+    // o and down. Per layer (both) against the tiles these replaced (64 x 64 up to 1024 columns, else 64 x 128 two a
+    // CU), us: 32 x 32 Qwen3-0.6B 31 tokens -8.3, 200 -9.1, Qwen3-4B 31 -128; 64 x 32 Qwen3-0.6B 512 -4.5, Qwen3-8B 100
+    // -130; 64 x 64 Qwen3-4B 333 -100; 128 x 64 Qwen3-4B 700 -74; 128 x 128 Qwen3-4B 1024 -35, Qwen3-8B 2000 -78 (two
+    // whole rounds). At 1.25 rounds (Qwen3-4B 2048) 128 x 128 loses 53 to 64 x 128.
+    if (g.al == nullptr && g.K % 64 == 0) {
+      if (deep && blocks(32, 32) <= 256) return launch_split_cfg<EPI, 32, 32, 8, 1, 128, false, 1, 1, 4>(g, s);
+      if (deep && blocks(64, 32) <= 256) return launch_split_cfg<EPI, 64, 32, 3, 2, 128, false, 2, 1, 4>(g, s);
+      if (deep && blocks(64, 64) <= 256) return launch_split_cfg<EPI, 64, 64, 4, 1, 128, false, 2, 2>(g, s);
+      if (!deep && blocks(128, 64) < 256) return launch_split_cfg<EPI, 64, 64, 3, 3, 64, false>(g, s);
+      if (blocks(128, 64) <= 256) return launch_split_cfg<EPI, 128, 64, 4, 1, 64, false, 4, 2>(g, s);
+      const int b = blocks(128, 128);
+      if (b <= 256 || 5 * b >= 4 * 256 * rounds(b, 256)) return launch_split_cfg<EPI, 128, 128, 4, 1, 64, false, 4, 2>(g, s);
+    }
+  }
+  if constexpr (EPI == EPI_STORE) {  // the batch's LM head: the large QKV tile
+    if (g.al != nullptr && g.M > 64 && blocks(128, 128) >= 512)
+      return launch_split_cfg<EPI, 128, 128, 3, 2, 32, true, 4, 2>(g, s);
   }
   // 64 x 128 tiles, two blocks per CU: 64-deep slices in a 2-slot ring, or 32-deep ones in a 4-slot ring when K
-  // is not a multiple of 64 (measured on the Qwen3-0.6B prefill shapes at 2048 tokens). The residual projections
-  // of <= 1024 columns (o and down) would get one 64 x 128 tile per CU; 64 x 64 tiles, up to three blocks per CU,
-  // give them twice the blocks (2048 tokens: 8.29 -> 7.97 ms per prefill); on single fp16 activations a 3-slot ring
-  // fits three blocks per CU and hides more of the load latency (6.92 -> 6.69 ms)
+  // is not a multiple of 64; o and down with hi/lo activations of up to 1024 columns 64 x 64 tiles (twice the blocks)
   if constexpr (EPI == EPI_RESIDUAL) {
-    if (g.K % 64 == 0 && g.N <= 1024) {
-      if (g.al == nullptr && mt128 * ((g.N + 63) / 64) >= 256)
-        return launch_split_cfg<EPI, 128, 64, 4, 1, 64, false, 4, 2>(g, s);
-      return g.al != nullptr ? launch_split_cfg<EPI, 64, 64, 2, 3, 64, true>(g, s)
-                             : launch_split_cfg<EPI, 64, 64, 3, 3, 64, false>(g, s);
-    }
+    if (g.al != nullptr && g.K % 64 == 0 && g.N <= 1024) return launch_split_cfg<EPI, 64, 64, 2, 3, 64, true>(g, s);
   }
   if (g.al != nullptr)
     return g.K % 64 == 0 ? launch_split_cfg<EPI, 64, 128, 2, 2, 64, true>(g, s)

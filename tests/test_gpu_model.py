@@ -159,6 +159,39 @@ def test_prefill_split_gemm_matches_staged_kernel(gpu_ctx, monkeypatch, n, hilo)
         m.close()
 
 
+@pytest.mark.parametrize("shape, ns", [
+    ((1024, 3072, 16, 8), (31, 32, 33, 65, 129, 257, 513, 1025)),
+    ((2560, 9728, 32, 8), (31, 64, 129, 321, 700, 1030)),
+    ((960, 2880, 8, 4), (33, 700)),  # K a multiple of 64, not of 128
+    ((992, 3040, 2, 1), (65, 300)),  # hidden a multiple of 32 only
+], ids=lambda v: f"{v[0]}x{v[1]}" if len(v) == 4 else "")
+def test_prefill_gemm_tiles_match_staged_kernel(gpu_ctx, monkeypatch, shape, ns):
+    """Every tile that the number of blocks selects (32 x 32 to 128 x 128 for o and down, 32 x 64 to 256 x 192 for
+    gate/up, 32, 64 and 128 rows for QKV; loader waves; 128-deep slices) accumulates the products of the register-staged
+    kernel in its order: logits bit-identical, at row counts on and off the edges of the tiles."""
+    monkeypatch.delenv("SOC_PREFILL_SPLIT", raising=False)
+    hidden, inter, nq, nkv = shape
+    cfg = S.QwenConfig(vocab_size=128, hidden_size=hidden, num_hidden_layers=1, num_attention_heads=nq,
+                       num_key_value_heads=nkv, intermediate_size=inter, tie_word_embeddings=True)
+    m = _gpu_model(gpu_ctx, cfg, S.synth_weights(cfg, 31))
+    kv = S.KVCache(m, 1, max(ns) + 8)
+    try:
+        for n in ns:
+            ids = S.synth_tokens(n, "tiles", cfg.vocab_size, n)
+            runs = []
+            for staged in (True, False):
+                if staged:
+                    monkeypatch.setenv("SOC_PREFILL_GEMM", "staged")
+                else:
+                    monkeypatch.delenv("SOC_PREFILL_GEMM", raising=False)
+                kv.reset(0)
+                runs.append(S.prefill(m, kv, 0, ids, 0, logit_rows=n)[0])
+            np.testing.assert_array_equal(runs[1], runs[0], err_msg=f"{n} tokens")
+    finally:
+        kv.close()
+        m.close()
+
+
 def test_decode_steps_equal_decode_loop(gpu_ctx):
     cfg, seed, _, _ = SMALL_MODELS["tiny_untied"]
     m = _gpu_model(gpu_ctx, cfg, S.synth_weights(cfg, seed))
