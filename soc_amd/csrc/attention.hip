@@ -28,23 +28,42 @@ constexpr int kMaxCombine = 160;  // key chunks one attention row may be split i
 // number of chunks however ragged the rows are. (With the chunk index fastest, rows of few chunks would load only
 // the XCDs and shader engines that low chunk indices map to.)
 // PAIR: outputs as hi/lo pairs (out_hi, out_lo) instead of fp32.
-template <int G, bool FUSED, int KH, bool PAIR>
-__global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
-  __shared__ float qs[G][HD];
-  __shared__ float kn[HD], vn[HD];
-  __shared__ float sc[G][256];
-  __shared__ float red[4][G][HD];
-  __shared__ float mstat[G], lstat[G];
-  __shared__ float cm[G][kMaxCombine], cl[G][kMaxCombine];  // split combine: chunk maxima / weights, sums
-  __shared__ int last;
+// 16-byte members: they are read four floats at a time
+template <int G>
+struct AttnLds {
+  alignas(16) float qs[G][HD];
+  alignas(16) float kn[HD];
+  alignas(16) float vn[HD];
+  alignas(16) float sc[G][256];
+  alignas(16) float red[4][G][HD];
+  alignas(16) float cm[G][kMaxCombine];  // split combine: chunk maxima / weights
+  alignas(16) float cl[G][kMaxCombine];  // and sums
+  float mstat[G], lstat[G];
+  int last;
+};
+
+// One block's work. NT key tiles of 16 per wave, so chunks of 64 NT keys: with NT = 4 the values are requested
+// after the scores, into the keys' registers; with fewer tiles (single-sequence decode of a long row) every wave has
+// keys to load and the values are in flight with them, one memory round trip for the chunk. KH = 2: the keys and the
+// values in two halves each (half the registers, so more blocks per CU; a second round trip for each).
+template <int G, bool FUSED, int KH, bool PAIR, int NT>
+__device__ __forceinline__ void attention_block(const AttnArgs& a, int qpos, AttnLds<G>& lds) {
+  constexpr int chunk = 64 * NT;
+  static_assert(NT == 4 || KH == 1, "halves only of whole chunks");
+  auto& qs = lds.qs;
+  auto& kn = lds.kn;
+  auto& vn = lds.vn;
+  auto& sc = lds.sc;
+  auto& red = lds.red;
+  auto& mstat = lds.mstat;
+  auto& lstat = lds.lstat;
+  auto& cm = lds.cm;
+  auto& cl = lds.cl;
+  int& last = lds.last;
 
   const int b = blockIdx.z, g = blockIdx.x, s = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int qpos = (a.pos != nullptr ? a.pos[b] : b) + a.pos_base;
   const int S = qpos + 1;
-  // up to 256 keys one block per (row, KV head) takes them all (no partials and no combine); longer rows use the
-  // caller's chunk (single-sequence decode splits them finer than 256 for more blocks)
-  const int chunk = S <= 256 ? 256 : a.chunk;
   const int nact = (S + chunk - 1) / chunk;
   if (s >= nact) return;
   const int slot = a.slot != nullptr ? a.slot[b] : a.slot_base;
@@ -56,26 +75,36 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
   const int c0 = s * chunk;
   const int n = min(chunk, S - c0);
 
-  // The chunk's keys, as MFMA B operands: the wave's keys are 64 w .. 64 w + 63 of the chunk; lane (key kl, group kg)
+  // The chunk's keys, as MFMA B operands: the wave's keys are 16 NT w .. of the chunk; lane (key kl, group kg)
   // = (lane % 16, lane / 16) holds the 16 bytes of dims 32 t + 8 kg of its key for t = 0..3, as stored (fp16 keys are
   // exact). Keys past the chunk's end load the last key (their scores are never stored), so the loads need no
   // branch. They are issued right after the query's own loads; loads complete in issue order, so the staging waits
   // for the query only and the keys stay in flight.
   const int kl = lane & 15, kg = lane >> 4;
-  // KH = 2: the keys and the values in two halves each (half the registers, so more blocks per CU; a second round
-  // trip for each)
-  constexpr int T4H = 4 / KH, UH = 16 / KH;
-  u32x4 raw[16 / KH];  // keys: [tile t4][dim step t] -> raw[4 (t4 % T4H) + t]; values: the row layout below
+  constexpr int T4H = NT / KH, UH = 4 * NT / KH;
+  u32x4 raw[4 * NT / KH];  // keys: [tile t4][dim step t] -> raw[4 (t4 % T4H) + t]; values: the row layout below
+  u32x4 rawv[NT < 4 ? 4 * NT : 1];  // values in flight with the keys
   // keys and values stream past the caches (each is read once per step: 4.05 -> 4.02 ms per Qwen3-4B x 16 ragged
   // step, 1.99 -> 1.98 ms per Qwen3-4B batch-1 token)
   auto kv_load = [](const f16* p) { return load_stream16(p); };
   auto load_keys = [&](int h) {
 #pragma unroll
     for (int t4 = h * T4H; t4 < (h + 1) * T4H; ++t4) {
-      const int p = min(64 * wid + 16 * t4 + kl, n - 1);
+      const int p = min(16 * NT * wid + 16 * t4 + kl, n - 1);
 #pragma unroll
       for (int t = 0; t < 4; ++t)
         raw[4 * (t4 - h * T4H) + t] = kv_load(kb + static_cast<size_t>(c0 + p) * HD + 32 * t + 8 * kg);
+    }
+  };
+
+  const int sub = lane & 15, r = lane >> 4;
+  auto load_values = [&](int h) {  // (keys past the chunk's end load the last one, never used)
+#pragma unroll
+    for (int u = h * UH; u < (h + 1) * UH; ++u) {
+      const int p = min(u * 16 + wid * 4 + r, n - 1);
+      const u32x4 v = kv_load(vb + static_cast<size_t>(c0 + p) * HD + sub * 8);
+      if constexpr (NT < 4) rawv[u] = v;
+      else raw[u - h * UH] = v;
     }
   };
 
@@ -98,6 +127,7 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
     const float rs = a.rope_sin[static_cast<size_t>(qpos) * (HD / 2) + lane];
     __builtin_amdgcn_sched_barrier(0);
     load_keys(0);
+    if constexpr (NT < 4) load_values(0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < NV; ++t) {
@@ -134,6 +164,7 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
     for (int u = 0; u < QN; ++u) qv[u] = row[(g * G) * HD + min(tid + 256 * u, G * HD - 1)];
     __builtin_amdgcn_sched_barrier(0);
     load_keys(0);
+    if constexpr (NT < 4) load_values(0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < QN; ++u) {
@@ -143,7 +174,6 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
   }
   __syncthreads();
 
-  const int sub = lane & 15, r = lane >> 4;
   auto put = [&](int j, int i, float o) {  // one output of query head j
     const size_t at = static_cast<size_t>(b) * a.ld_out + (g * G + j) * HD + i;
     if constexpr (PAIR) {
@@ -178,11 +208,11 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
     }
   }
 #pragma unroll
-  for (int t4 = 0; t4 < 4; ++t4) {
-    if (64 * wid + 16 * t4 >= n) break;  // wave-uniform: no key of this tile is in the chunk
+  for (int t4 = 0; t4 < NT; ++t4) {
+    if (16 * NT * wid + 16 * t4 >= n) break;  // wave-uniform: no key of this tile is in the chunk
     if (KH == 2 && t4 == T4H) load_keys(1);
     const int ri = 4 * (t4 % T4H);
-    const int p = 64 * wid + 16 * t4 + kl;
+    const int p = 16 * NT * wid + 16 * t4 + kl;
     if (FUSED && c0 + p == qpos) {  // the new key: from this kernel's own normed and roped copy
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
@@ -217,14 +247,7 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
         for (int j = 0; j < G; ++j) sc[j][p] = (d[j] + d[G + j] * (1.0f / 2048.0f)) * a.scale;
     }
   }
-  auto load_values = [&](int h) {  // (keys past the chunk's end load the last one, never used)
-#pragma unroll
-    for (int u = h * UH; u < (h + 1) * UH; ++u) {
-      const int p = min(u * 16 + wid * 4 + r, n - 1);
-      raw[u - h * UH] = kv_load(vb + static_cast<size_t>(c0 + p) * HD + sub * 8);
-    }
-  };
-  load_values(0);
+  if constexpr (NT == 4) load_values(0);
   __syncthreads();
 
   // softmax statistics per query head
@@ -253,7 +276,7 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[j][i] = 0.0f;
 #pragma unroll
-  for (int u = 0; u < 16; ++u) {
+  for (int u = 0; u < 4 * NT; ++u) {
     const int p = u * 16 + wid * 4 + r;
     if (u * 16 >= n) break;
     if (KH == 2 && u == UH) load_values(1);
@@ -263,7 +286,8 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) vf[i] = vn[sub * 8 + i];
       } else {
-        f16x8_to_f32(raw[u % UH], vf);
+        if constexpr (NT < 4) f16x8_to_f32(rawv[u], vf);
+        else f16x8_to_f32(raw[u % UH], vf);
       }
 #pragma unroll
       for (int j = 0; j < G; ++j) {
@@ -375,6 +399,25 @@ __global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
     put(j, i, O / lstat[j]);
   }
   if (tid == 0) st_dev(a.counters + b * a.nkv + g, 0);
+}
+
+// FINE (single-sequence decode): chunks by the row's length (a.chunk = 0, attn_row_chunk) or of a.chunk keys (against
+// chunks of 64 keys beyond 256 and one chunk up to that, keys and values one after the other: 4071 keys of 32 query and
+// 8 KV heads 34.0 -> 27.4 us a call, Qwen3-4B decode with 2900 keys -7 %, 200 keys -1 %). Otherwise (rows of a batch,
+// blocks enough) chunks of 256.
+template <int G, bool FUSED, int KH, bool PAIR, bool FINE>
+__global__ __launch_bounds__(256) void k_attention(AttnArgs a) {
+  __shared__ AttnLds<G> lds;
+  const int b = blockIdx.z;
+  const int qpos = (a.pos != nullptr ? a.pos[b] : b) + a.pos_base;
+  if constexpr (FINE) {
+    const int chunk = a.chunk != 0 ? a.chunk : attn_row_chunk(qpos + 1);
+    if (chunk == 256) attention_block<G, FUSED, KH, PAIR, 4>(a, qpos, lds);
+    else if (chunk == 64) attention_block<G, FUSED, 1, PAIR, 1>(a, qpos, lds);
+    else attention_block<G, FUSED, 1, PAIR, 2>(a, qpos, lds);
+  } else {
+    attention_block<G, FUSED, KH, PAIR, 4>(a, qpos, lds);
+  }
 }
 
 // grid = (T, nq + nkv), block = 64: one wave per (row, head). q heads -> q_out; k heads -> cache (and v copy).
@@ -1100,25 +1143,29 @@ bool attention_prefill_mfma_supported(int nq, int nkv) {
 
 hipError_t launch_attention(const AttnArgs& a, int fused, hipStream_t s) {
   const int G = a.nq / a.nkv;
-  if (a.chunk > 256 || a.chunk <= 0) return hipErrorInvalidValue;
+  if (a.chunk != 64 && a.chunk != 128 && a.chunk != 256 && a.chunk != 0) return hipErrorInvalidValue;
+  if (a.out_hi != nullptr && a.chunk != 256) return hipErrorInvalidValue;
   if (a.max_split > kMaxCombine) return hipErrorInvalidValue;
   if (a.out_hi != nullptr ? a.out_lo == nullptr || fused : a.out == nullptr) return hipErrorInvalidValue;
   const dim3 grid(a.nkv, a.max_split, a.B), block(256);
-  // unfused rows (the ragged batch): keys and values in halves, 88 instead of 112 registers, five blocks per CU
-  // instead of four (Qwen3-4B x 16 ragged step 4.07 -> 4.04 ms); the fused single-sequence decode runs few blocks and
-  // keeps the one round trip per operand
-#define SOC_ATTN_CASE(GG)                                                                  \
-  if (G == GG) {                                                                          \
-    if (fused) hipLaunchKernelGGL((k_attention<GG, true, 1, false>), grid, block, 0, s, a);             \
-    else if (a.out_hi != nullptr) hipLaunchKernelGGL((k_attention<GG, false, 2, true>), grid, block, 0, s, a); \
-    else hipLaunchKernelGGL((k_attention<GG, false, 2, false>), grid, block, 0, s, a);                  \
-    return hipGetLastError();                                                             \
+  // whole chunks of unfused rows (the ragged batch): keys and values in halves, 88 instead of 112 registers, five
+  // blocks per CU instead of four (Qwen3-4B x 16 ragged step 4.07 -> 4.04 ms); the fused single-sequence decode runs
+  // few blocks and keeps the one round trip per operand
+#define SOC_ATTN_LAUNCH(...) hipLaunchKernelGGL((k_attention<__VA_ARGS__>), grid, block, 0, s, a)
+#define SOC_ATTN_CASE(GG)                                                          \
+  if (G == GG) {                                                                   \
+    if (fused) SOC_ATTN_LAUNCH(GG, true, 1, false, true);                          \
+    else if (a.out_hi != nullptr) SOC_ATTN_LAUNCH(GG, false, 2, true, false);      \
+    else if (a.chunk < 256) SOC_ATTN_LAUNCH(GG, false, 2, false, true);            \
+    else SOC_ATTN_LAUNCH(GG, false, 2, false, false);                              \
+    return hipGetLastError();                                                      \
   }
   SOC_ATTN_CASE(1)
   SOC_ATTN_CASE(2)
   SOC_ATTN_CASE(4)
   SOC_ATTN_CASE(8)
 #undef SOC_ATTN_CASE
+#undef SOC_ATTN_LAUNCH
   return hipErrorInvalidValue;
 }
 

@@ -94,9 +94,28 @@ struct AttnArgs {
   f16* out_lo;
   float* part;           // split partials [B][nq][max_split][d + 2]
   int* counters;         // [B][nkv] zero-initialised
-  int B, nq, nkv, max_split, chunk;
+  int B, nq, nkv, max_split;
+  int chunk;             // keys per chunk: 64, 128 or 256; 0 (single-sequence decode): attn_row_chunk of the row's length
   float scale;
 };
+// Keys per chunk of a single-sequence decode row of S keys. One block takes a row of up to 160; beyond, short chunks
+// give a row more blocks (every block is one chunk of one KV head) until their partial sums cost more than they save.
+// soc_attention_decode, 32 query and 8 KV heads, us per call at 64 / 128 / 256 keys: 64 keys 18.6 / 19.1 / 19.4, 128
+// keys 21.6 / 20.1 / 20.3, 256 keys 21.5 / 23.0 / 22.5, 1024 keys 22.6 / 23.4 / 25.7, 1500 keys 24.7 / 23.6 / 25.6, 3000
+// keys 29.2 / 26.3 / 26.2, 8000 keys 45.8 / 33.9 / 30.1 (inside the layers of a decode step 128 at 65 to 128 keys is
+// slower than 256, by 0.3 us a layer).
+__host__ __device__ inline int attn_row_chunk(int S) {
+  return S <= 64 ? 64 : S <= 160 ? 256 : S <= 1024 ? 64 : S <= 3072 ? 128 : 256;
+}
+// Most chunks any such row of up to `cap` keys has.
+inline int attn_row_splits(int cap) {
+  int n = (cap + 255) / 256;
+  for (int S : {cap < 1024 ? cap : 1024, cap < 3072 ? cap : 3072}) {
+    const int k = (S + attn_row_chunk(S) - 1) / attn_row_chunk(S);
+    n = k > n ? k : n;
+  }
+  return n;
+}
 // fused = 1: q/k norm + RoPE + KV append of the new token are done inside (decode).
 hipError_t launch_attention(const AttnArgs& a, int fused, hipStream_t s);
 // Prefill chunk (pos == slot == nullptr) on MFMA: causal over keys 0..pos_base+row of the slot's cache, which must

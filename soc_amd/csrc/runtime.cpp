@@ -130,17 +130,20 @@ constexpr int kAttnChunk = 256;
 // next token's first layer streams while the last layer of the current one runs).
 constexpr int kXcdStepsPerLaunch = 128;
 
-// Keys per attention chunk of single-sequence per-op decode for a cache of `cap` positions: the smallest of 64, 128,
-// 256 that keeps a full cache within 160 chunks (the kernel's combine limit). Smaller chunks give a short context
-// more blocks (at batch 1 every block is one chunk of one KV head). SOC_DECODE_CHUNK overrides (64, 128 or 256).
+// Keys per attention chunk of single-sequence per-op decode: 0, by the row's length (soc::attn_row_chunk), or what
+// SOC_DECODE_CHUNK says (64, 128 or 256, where a full cache of `cap` positions then has at most 160 chunks, the kernel's
+// combine limit).
 int decode_attn_chunk(int cap) {
   if (const char* e = std::getenv("SOC_DECODE_CHUNK")) {
     const int v = std::atoi(e);
     if ((v == 64 || v == 128 || v == 256) && (cap + v - 1) / v <= 160) return v;
   }
-  for (int c = 64; c < kAttnChunk; c *= 2)
-    if ((cap + c - 1) / c <= 160) return c;
-  return kAttnChunk;
+  return 0;
+}
+// Most chunks a row of up to `cap` keys has then.
+int decode_attn_splits(int cap) {
+  const int chunk = decode_attn_chunk(cap);
+  return chunk != 0 ? (cap + chunk - 1) / chunk : soc::attn_row_splits(cap);
 }
 constexpr int kQChunk = 8;  // rows per group-quantized projection call in a quantized model's prefill (k_qmm M <= 8)
 constexpr int kMaxBatchRows = 1024;
@@ -259,7 +262,7 @@ int check_config(const soc_qwen_config& c) {
 
 int ensure_decode_ws(soc_model* m, int cap) {
   DecodeWs& w = m->dws;
-  const int need_split = (cap + decode_attn_chunk(cap) - 1) / decode_attn_chunk(cap);
+  const int need_split = decode_attn_splits(cap);
   if (w.ready && w.max_split >= need_split && w.ring_cap >= cap) return SOC_OK;
   hipError_t se = hipStreamSynchronize(m->ctx->stream);
   if (se != hipSuccess) return hip_fail(se, "hipStreamSynchronize");
@@ -489,7 +492,7 @@ int enqueue_decode(soc_model* m, soc_kv* kv, int slot, const int32_t* d_slot) {
         a.counters = w.attn_counters;
         a.B = 1;
         a.chunk = decode_attn_chunk(kv->cap);
-        a.max_split = (kv->cap + a.chunk - 1) / a.chunk;
+        a.max_split = decode_attn_splits(kv->cap);
         const hipError_t ea = soc::launch_attention(a, 1, s);
         return ea == hipSuccess ? SOC_OK : hip_fail(ea, "attention decode");
       };
@@ -521,7 +524,7 @@ int enqueue_decode(soc_model* m, soc_kv* kv, int slot, const int32_t* d_slot) {
       a.counters = w.attn_counters;
       a.B = 1;
       a.chunk = decode_attn_chunk(kv->cap);
-      a.max_split = (kv->cap + a.chunk - 1) / a.chunk;
+      a.max_split = decode_attn_splits(kv->cap);
       if ((e = soc::launch_attention(a, 1, s)) != hipSuccess) return hip_fail(e, "attention decode");
       g = soc::GemvArgs{};
       g.x = w.attn;
@@ -2602,7 +2605,8 @@ int soc_attention_decode(soc_ctx* ctx, const float* q, const void* keys, const v
   a.B = 1;
   a.nq = nq;
   a.nkv = nkv;
-  a.chunk = decode_attn_chunk(cap);
+  const int chunk = decode_attn_chunk(cap);
+  a.chunk = chunk != 0 ? chunk : soc::attn_row_chunk(kv_len);
   a.max_split = (kv_len + a.chunk - 1) / a.chunk;
   a.scale = 1.0f / std::sqrt(128.0f);
   if (a.max_split > 160) return soc::fail(SOC_ERR_INVALID, "attention: too many keys for the capacity's chunk size");

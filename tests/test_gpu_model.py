@@ -192,6 +192,35 @@ def test_prefill_gemm_tiles_match_staged_kernel(gpu_ctx, monkeypatch, shape, ns)
         m.close()
 
 
+@pytest.mark.parametrize("bits", [0, 4])
+def test_decode_attention_chunk_edges(gpu_ctx, monkeypatch, bits):
+    """Per-op decode at the edges of its attention chunks (one launch on any length: the chunk is picked on the device
+    from the row's) gives the logits of the prefill that holds the same row, as in test_decode_matches_prefill_rows."""
+    monkeypatch.setenv("SOC_DECODE", "graph")
+    monkeypatch.delenv("SOC_DECODE_CHUNK", raising=False)
+    cfg = S.QwenConfig(vocab_size=128, hidden_size=256, num_hidden_layers=2, num_attention_heads=8,
+                       num_key_value_heads=2, intermediate_size=512, tie_word_embeddings=True)
+    m = _gpu_model(gpu_ctx, cfg, S.synth_weights(cfg, 61))
+    if bits:
+        m.quantize(bits)
+    n = 3076 if not bits else 260
+    ids = S.synth_tokens(62, "edges", cfg.vocab_size, n)
+    kv = S.KVCache(m, 1, n + 8)
+    try:
+        full, _ = S.prefill(m, kv, 0, ids, 0, logit_rows=n)
+        for p in (1, 62, 63, 64, 126, 127, 128, 191, 192, 255, 256, 1022, 1023, 1024, 3070, 3071, 3072):
+            if p + 3 > n:
+                break
+            kv.reset(0)
+            S.prefill(m, kv, 0, ids[:p], 0, logit_rows=0)
+            for t in range(p, p + 2):
+                lg, _ = S.decode(m, kv, 0, int(ids[t]))
+                assert_logits_close(lg, full[t], f"row {t}")
+    finally:
+        kv.close()
+        m.close()
+
+
 def test_decode_steps_equal_decode_loop(gpu_ctx):
     cfg, seed, _, _ = SMALL_MODELS["tiny_untied"]
     m = _gpu_model(gpu_ctx, cfg, S.synth_weights(cfg, seed))

@@ -217,6 +217,38 @@ def test_attention_decode_matches_oracle(gpu_ctx, oracle_mod, heads):
             gpu_ctx.free(p)
 
 
+@pytest.mark.parametrize("heads", [(16, 8), (32, 8), (8, 1), (8, 8)])
+@pytest.mark.parametrize("chunk", [None, "64", "128", "256"])
+def test_attention_decode_chunk_edges(gpu_ctx, monkeypatch, heads, chunk):
+    """Key counts at the edges of the chunks (one, two and four key tiles a wave) and of the rule that picks them by
+    length, against float64. Scores come from query halves exact to 2^-22 and fp32 sums of 128 products (error below
+    2e-6 at |score| < 6), which moves an average of values |v| < 5 by at most 2 x 2e-6 x 5."""
+    if chunk is None:
+        monkeypatch.delenv("SOC_DECODE_CHUNK", raising=False)
+    else:
+        monkeypatch.setenv("SOC_DECODE_CHUNK", chunk)
+    nq, nkv = heads
+    cap = 3200
+    rng = np.random.default_rng(nq + 5 * nkv)
+    k, v = _kv_planes(rng, nkv, cap)
+    pk, pv = gpu_ctx.upload(k), gpu_ctx.upload(v)
+    pq, po = gpu_ctx.alloc(nq * 128 * 4), gpu_ctx.alloc(nq * 128 * 4)
+    kd, vd = k.astype(np.float64), v.astype(np.float64)
+    try:
+        for s_len in (1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 193, 255, 256, 257, 1024, 1025, 3072, 3073, 3200):
+            q = rng.standard_normal((1, nq, 128)).astype(np.float32)
+            gpu_ctx.write(pq, q)
+            S.attention_decode(gpu_ctx, pq, pk, pv, po, s_len, nq, nkv, cap)
+            out = gpu_ctx.download(po, q.shape, np.float32)
+            sc = np.einsum("gjd,gpd->gjp", q.astype(np.float64).reshape(nkv, -1, 128), kd[:, :s_len]) / np.sqrt(128.0)
+            w = np.exp(sc - sc.max(-1, keepdims=True))
+            ref = np.einsum("gjp,gpd->gjd", w / w.sum(-1, keepdims=True), vd[:, :s_len]).reshape(q.shape)
+            np.testing.assert_allclose(out, ref, rtol=0, atol=2e-5, err_msg=f"{s_len} keys")
+    finally:
+        for p in (pk, pv, pq, po):
+            gpu_ctx.free(p)
+
+
 # ---- the reference's fp32 op kernels ----
 
 def _run(ctx, fn, *args):
