@@ -624,11 +624,14 @@ hipError_t launch_split_epi(const GemmSplitArgs& g, hipStream_t s) {
       if (c128 <= c64) return launch_split_cfg<EPI, 128, 128, 2, 2, 64, false, 4, 2>(g, s);
     }
   }
-  if constexpr (EPI == EPI_RESIDUAL) {
-    // o and down. Per layer (both) against the tiles these replaced (64 x 64 up to 1024 columns, else 64 x 128 two a
+  if constexpr (EPI == EPI_RESIDUAL || EPI == EPI_STORE) {
+    // o and down (and soc_gemm_f16). Per layer (both) against the tiles these replaced (64 x 64 up to 1024 columns, else 64 x 128 two a
     // CU), us: 32 x 32 Qwen3-0.6B 31 tokens -8.3, 200 -9.1, Qwen3-4B 31 -128; 64 x 32 Qwen3-0.6B 512 -4.5, Qwen3-8B 100
     // -130; 64 x 64 Qwen3-4B 333 -100; 128 x 64 Qwen3-4B 700 -74; 128 x 128 Qwen3-4B 1024 -35, Qwen3-8B 2000 -78 (two
-    // whole rounds). At 1.25 rounds (Qwen3-4B 2048) 128 x 128 loses 53 to 64 x 128.
+    // whole rounds). At 1.25 rounds (Qwen3-4B 2048) 128 x 128 loses 53 to 64 x 128, and so it does on rows that fill
+    // one 64-row tile. soc_gemm_f16, us a call: 31 x 4096 x 4096 47.2 -> 27.5, 128 x 2560 x 9728 93.8 -> 55.2, 2048 x 4096
+    // x 12288 298 -> 259 (31 x 151936 x 1024: 75.7, 88.9 with 128 x 128; 4096 x 4096 x 4096, four rounds of short K:
+    // 187, 193 with it).
     if (g.al == nullptr && g.K % 64 == 0) {
       if (deep && blocks(32, 32) <= 256) return launch_split_cfg<EPI, 32, 32, 8, 1, 128, false, 1, 1, 4>(g, s);
       if (deep && blocks(64, 32) <= 256) return launch_split_cfg<EPI, 64, 32, 3, 2, 128, false, 2, 1, 4>(g, s);
@@ -636,7 +639,8 @@ hipError_t launch_split_epi(const GemmSplitArgs& g, hipStream_t s) {
       if (!deep && blocks(128, 64) < 256) return launch_split_cfg<EPI, 64, 64, 3, 3, 64, false>(g, s);
       if (blocks(128, 64) <= 256) return launch_split_cfg<EPI, 128, 64, 4, 1, 64, false, 4, 2>(g, s);
       const int b = blocks(128, 128);
-      if (b <= 256 || 5 * b >= 4 * 256 * rounds(b, 256)) return launch_split_cfg<EPI, 128, 128, 4, 1, 64, false, 4, 2>(g, s);
+      if (g.M > 64 && (b <= 256 || (5 * b >= 4 * 256 * rounds(b, 256) && (b <= 512 || g.K >= 8192))))
+        return launch_split_cfg<EPI, 128, 128, 4, 1, 64, false, 4, 2>(g, s);
     }
   }
   if constexpr (EPI == EPI_STORE) {  // the batch's LM head: the large QKV tile

@@ -162,6 +162,25 @@ def test_gemm_f16_ragged_shapes_and_bad_operands(gpu_ctx, oracle_mod):
 
 # ---- attention ----
 
+@pytest.mark.parametrize("n, k", [(1024, 2048), (2560, 1024), (1000, 1088), (4100, 256), (130, 96)])
+def test_gemm_f16_rows_do_not_depend_on_the_tile(gpu_ctx, n, k):
+    """The tile follows the number of blocks, and every tile sums a row's products in one order: the rows of a call of
+    few rows are those of a call of many, bit for bit."""
+    rng = np.random.default_rng(n + k)
+    x = rng.standard_normal((1500, k)).astype(np.float16)
+    w = rng.standard_normal((n, k)).astype(np.float16)
+    px, pw, py = gpu_ctx.upload(x), gpu_ctx.upload(w), gpu_ctx.alloc(1500 * n * 4)
+    try:
+        S.gemm_f16(gpu_ctx, px, pw, py, 1500, n, k)
+        full = gpu_ctx.download(py, (1500, n), np.float32)
+        for m in (1, 31, 33, 64, 65, 129, 300, 513, 1025):
+            S.gemm_f16(gpu_ctx, px, pw, py, m, n, k)
+            np.testing.assert_array_equal(gpu_ctx.download(py, (m, n), np.float32), full[:m], err_msg=f"{m} rows")
+    finally:
+        for p in (px, pw, py):
+            gpu_ctx.free(p)
+
+
 def _kv_planes(rng, nkv, cap):
     k = rng.standard_normal((nkv, cap, 128)).astype(np.float16)
     v = rng.standard_normal((nkv, cap, 128)).astype(np.float16)
