@@ -163,6 +163,9 @@ hipError_t launch_kv_append_rows(const void* keys, const void* values, bool fp16
 
 // Token ids in device memory [n] -> dst [n], ids outside [0, vocab) replaced by 0 with *err set to 1 (ops.hip).
 hipError_t launch_stage_ids(const int32_t* src, int n, int vocab, int32_t* dst, int* err, hipStream_t s);
+// A batch step's rows from pinned host memory [ids | slots | positions] of n each (ops.hip).
+hipError_t launch_stage_batch(const int32_t* host, int n, int32_t* ids, int32_t* slots, int32_t* pos, int32_t* start,
+                              hipStream_t s);
 // A decode step's inputs in one launch: state[0] = dev_last ? *dev_last (checked like launch_stage_ids) : host_last,
 // state[1] = pos, *ring = 0 (ops.hip).
 hipError_t launch_decode_prologue(const int32_t* dev_last, int32_t host_last, int32_t pos, int vocab, int32_t* state,

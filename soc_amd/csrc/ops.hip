@@ -212,6 +212,18 @@ __global__ __launch_bounds__(256) void k_stage_ids(const int32_t* __restrict__ s
   }
 }
 
+// A batch step's rows, from three arrays of n in pinned host memory: token ids, slots, positions (= start).
+__global__ __launch_bounds__(256) void k_stage_batch(const int32_t* __restrict__ host, int n, int32_t* ids,
+                                                     int32_t* slots, int32_t* pos, int32_t* start) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int32_t id = host[i], slot = host[n + i], p = host[2 * n + i];
+  ids[i] = id;
+  slots[i] = slot;
+  pos[i] = p;
+  start[i] = p;
+}
+
 // A decode step's inputs: state[0] = the token (the host's, or the validated id at dev_last), state[1] = its
 // position, ring position 0.
 __global__ void k_decode_prologue(const int32_t* __restrict__ dev_last, int32_t host_last, int32_t pos, int vocab,
@@ -269,6 +281,12 @@ constexpr int64_t kMaxElems = int64_t{1} << 31;  // element counts the kernels i
 
 hipError_t launch_stage_ids(const int32_t* src, int n, int vocab, int32_t* dst, int* err, hipStream_t s) {
   hipLaunchKernelGGL(k_stage_ids, dim3(std::min(64, (n + 255) / 256)), dim3(256), 0, s, src, n, vocab, dst, err);
+  return hipGetLastError();
+}
+
+hipError_t launch_stage_batch(const int32_t* host, int n, int32_t* ids, int32_t* slots, int32_t* pos, int32_t* start,
+                              hipStream_t s) {
+  hipLaunchKernelGGL(k_stage_batch, dim3((n + 255) / 256), dim3(256), 0, s, host, n, ids, slots, pos, start);
   return hipGetLastError();
 }
 

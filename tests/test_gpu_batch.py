@@ -252,6 +252,33 @@ def test_batch_error_paths(gpu_ctx):
         m.close()
 
 
+def test_batch_rows_staged_through_pinned_memory(gpu_ctx):
+    """Calls of growing and shrinking row counts (the staging area is regrown, then used in part; counts around the
+    256 rows of a staging block): the returned tokens are the argmax of the returned logits, slots advance by one, and
+    a graph step run on a second cache from the same rows gives the same tokens."""
+    cfg = small_cfg()
+    m = S.Model(gpu_ctx, cfg).load(S.synth_weights(cfg, 71))
+    a, b = S.KVCache(m, 300, 16), S.KVCache(m, 300, 16)
+    rng = np.random.default_rng(72)
+    try:
+        for n in (2, 256, 257, 300, 3, 1):
+            slots = rng.permutation(300)[:n].astype(np.int32)
+            toks = rng.integers(0, cfg.vocab_size, n).astype(np.int32)
+            for i in range(300):
+                a.reset(i)
+                b.reset(i)
+            for step in range(2):
+                lg, nxt = S.decode_batch(m, a, slots, toks)
+                np.testing.assert_array_equal(nxt, np.argmax(lg, axis=1), err_msg=f"{n} rows")
+                assert all(a.length(int(i)) == step + 1 for i in slots)
+                np.testing.assert_array_equal(S.decode_batch_steps(m, b, slots, toks, 1)[0], nxt)
+                toks = nxt
+    finally:
+        a.close()
+        b.close()
+        m.close()
+
+
 @pytest.mark.parametrize("n", [17, 64, 65, 128, 130])
 def test_batch_row_gemm_edges(gpu_ctx, n):
     """The split-K row GEMMs of more than 16 rows at the edges of their 64- and 128-row tiles, widths off the 128-column
