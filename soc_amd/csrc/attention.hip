@@ -739,7 +739,8 @@ __global__ __launch_bounds__(256, 2) void k_attention_prefill_mfma(AttnArgs a) {
 
 // ------------------------------------------------------------------------------------------------------------
 // Causal GQA attention for a prefill chunk, balanced: a block takes two 32-row query tiles of one KV head, tile j
-// and tile nqt - 1 - j, one after the other, so every block sees about the same number of visible keys. Its 8 waves
+// and tile nqt - 1 - j, one after the other, so every block sees about the same number of visible keys (one tile, where
+// there are no more tiles than CUs). Its 8 waves
 // are HB query heads (the whole group of the KV head) x R = 8 / HB key residues: key tile kt goes to the waves of
 // residue kt % R, and each step stages R tiles. At the end of a query tile the R partial (max, sum, weighted values)
 // of each row are merged through LDS: every wave owns 4 / R of the four 32-dimension blocks of its head's output and
@@ -760,7 +761,7 @@ __global__ __launch_bounds__(256, 2) void k_attention_prefill_mfma(AttnArgs a) {
 // read ds_read_b64_tr_b16 (in each 16-lane group, lane j names 8 bytes = 4 dims of one key, and lane i receives dim
 // i of 4 consecutive keys), so no register staging or transposed stores are needed. Keys past the chunk's last row
 // read as zero (the buffer range ends there) and are masked (p = 0).
-// grid = ceil(ceil(B / 32) / 2) * nkv blocks (block b: KV head b % nkv, so with 8 KV heads each XCD's L2 holds one
+// grid = ceil(B / 32) or ceil(ceil(B / 32) / 2) times nkv blocks (block b: KV head b % nkv, so with 8 KV heads each XCD's L2 holds one
 // head), block = 512, dynamic LDS = [key/value ring | query rows], with the merge area over the ring (and past it
 // when it does not fit, in which case the query rows are not prefetched).
 // ------------------------------------------------------------------------------------------------------------
@@ -805,6 +806,7 @@ __global__ __launch_bounds__(512, 1) void k_attention_prefill_pairs(AttnArgs a) 
   const int ql = lane & 31, hb = lane >> 5;
   const int nqt = (a.B + 31) / 32;
   const int j = static_cast<int>(blockIdx.x / a.nkv);
+  const int partner = static_cast<int>(gridDim.x) == nqt * a.nkv ? j : nqt - 1 - j;  // j: the block has one tile
   const size_t head_base = static_cast<size_t>(a.slot_base) * a.slot_stride +
                            static_cast<size_t>(a.layer) * a.layer_stride + static_cast<size_t>(g) * a.cap * HD;
   const f16* kb = a.kcache + head_base;
@@ -833,8 +835,8 @@ __global__ __launch_bounds__(512, 1) void k_attention_prefill_pairs(AttnArgs a) 
   };
 
   for (int ph = 0; ph < 2; ++ph) {
-    if (ph == 1 && nqt - 1 - j == j) break;  // odd tile count: the middle tile has no partner
-    const int qt = ph == 0 ? j : nqt - 1 - j;
+    if (ph == 1 && partner == j) break;  // one tile a block, or the middle one of an odd count
+    const int qt = ph == 0 ? j : partner;
     const int t0 = qt * 32;
     const int t = t0 + ql;
     const int tq = min(t, a.B - 1);  // rows past the chunk compute a copy of the last row, never stored
@@ -887,9 +889,9 @@ __global__ __launch_bounds__(512, 1) void k_attention_prefill_pairs(AttnArgs a) 
         }
       }
     }
-    if (Lds::prefetch_q && ph == 0 && nqt - 1 - j != j) {
+    if (Lds::prefetch_q && ph == 0 && partner != j) {
       block_barrier();  // every wave has read its query rows: the partner tile's rows go to the same place
-      load_q(nqt - 1 - j);
+      load_q(partner);
     }
     // A operand of O^T = V^T . P^T for dims db*32.. and the 16-key step k2: lane (dim l % 32, hb) needs keys
     // hb*4 + 0..3 and 8 + hb*4 + 0..3 of the step (the key order of the P^T operand); 16-lane group grp covers dims
@@ -1090,8 +1092,13 @@ hipError_t launch_pairs_lo(const AttnArgs& a, hipStream_t s) {
       reinterpret_cast<const void*>(k_attention_prefill_pairs<HB, R, LOQ, LOP>), hipFuncAttributeMaxDynamicSharedMemorySize,
       static_cast<int>(lds));
   if (attr != hipSuccess) return attr;
+  // Pairs of tiles even out the blocks' work where there are more tiles than CUs. With fewer every tile has a CU of its
+  // own (a block's LDS fills one), and a pair would only put two behind each other: the keys of the past twice.
+  // soc_attention_prefill, 16 query and 8 KV heads, us a call: 100 rows after 1000 keys 50.9 -> 33.3, 333 after 700 46.3
+  // -> 32.6, 1000 after 1500 74.7 -> 53.6; 1000 rows of no past 37.8 -> 32.1.
   const int nqt = (a.B + 31) / 32;
-  hipLaunchKernelGGL((k_attention_prefill_pairs<HB, R, LOQ, LOP>), dim3(((nqt + 1) / 2) * a.nkv), dim3(512), lds, s, a);
+  const int per_head = nqt * a.nkv <= 256 ? nqt : (nqt + 1) / 2;
+  hipLaunchKernelGGL((k_attention_prefill_pairs<HB, R, LOQ, LOP>), dim3(per_head * a.nkv), dim3(512), lds, s, a);
   return hipGetLastError();
 }
 // SOC_PREFILL_ATTN_SPLIT=0: q and p as single fp16 values; =q: hi/lo for q only; =p: for p only

@@ -213,6 +213,31 @@ def test_attention_prefill_matches_oracle(gpu_ctx, oracle_mod, heads, rows, pos_
     _assert_close(out, ref, 3e-3, f"prefill attention {nq}q/{nkv}kv rows {rows} at {pos_base}")
 
 
+@pytest.mark.parametrize("heads, rows", [((16, 8), 1100), ((32, 8), 1057), ((8, 2), 4128)])
+def test_attention_prefill_one_tile_blocks(gpu_ctx, heads, rows):
+    """More query tiles of 32 rows than CUs: two tiles a block; up to as many: one. Calls of few rows (one tile, odd and
+    even counts, a ragged last one) give those rows of a call of many, bit for bit."""
+    nq, nkv = heads
+    past = 300
+    cap = past + rows
+    rng = np.random.default_rng(rows)
+    k, v = _kv_planes(rng, nkv, cap)
+    q = rng.standard_normal((rows, nq, 128)).astype(np.float32)
+    pk, pv = gpu_ctx.upload(k), gpu_ctx.upload(v)
+    pq, po = gpu_ctx.upload(q), gpu_ctx.alloc(q.nbytes)
+    try:
+        S.attention_prefill(gpu_ctx, pq, pk, pv, po, rows, past, nq, nkv, cap)
+        full = gpu_ctx.download(po, q.shape, np.float32)
+        for at, m in ((0, 32), (32, 64), (64, 95), (0, 1024 * 8 // nkv), (960, rows - 960)):
+            m = min(m, rows - at)
+            S.attention_prefill(gpu_ctx, pq + at * nq * 512, pk, pv, po, m, past + at, nq, nkv, cap)
+            out = gpu_ctx.download(po, (m, nq, 128), np.float32)
+            np.testing.assert_array_equal(out, full[at:at + m], err_msg=f"{m} rows from {at}")
+    finally:
+        for p in (pk, pv, pq, po):
+            gpu_ctx.free(p)
+
+
 @pytest.mark.parametrize("heads", [(16, 8), (32, 8), (8, 1), (8, 8)])
 def test_attention_decode_matches_oracle(gpu_ctx, oracle_mod, heads):
     nq, nkv = heads
