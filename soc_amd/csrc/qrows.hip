@@ -263,13 +263,15 @@ k_qrows(QRowsArgs a) {
         const int t = (first + (sl / TW) * static_cast<int>(gridDim.x)) * TW + sl % TW;
         if (sl < held * TW && t < ntiles && m < M && (EPI != EPI_SWIGLU || c < 8)) {
           const int n = t * TO + c;
-          float v = 0.0f, g = 0.0f;
+          // the waves' sums in float64: seven fp32 roundings of the whole result less
+          double vd = 0.0, gd = 0.0;
 #pragma unroll
-          for (int w = 0; w < KW; ++w) v += red[buf][sl][w][m][c];
+          for (int w = 0; w < KW; ++w) vd += static_cast<double>(red[buf][sl][w][m][c]);
           if constexpr (EPI == EPI_SWIGLU) {
 #pragma unroll
-            for (int w = 0; w < KW; ++w) g += red[buf][sl][w][m][c + 8];
+            for (int w = 0; w < KW; ++w) gd += static_cast<double>(red[buf][sl][w][m][c + 8]);
           }
+          const float v = static_cast<float>(vd), g = static_cast<float>(gd);
           if (n < nout) {
             const size_t o = static_cast<size_t>(m) * nout + n;
             if constexpr (EPI == EPI_SWIGLU) a.yh[o] = static_cast<f16>(silu_ref(v) * g);
@@ -285,6 +287,22 @@ k_qrows(QRowsArgs a) {
     if (AHEAD && nstep < nsteps) cur = nxt;
     step = nstep;
     pass = nps;
+  }
+}
+
+// group_sum<L> with the sums of 16 lanes added in float64 (two to four terms: one rounding instead of up to two levels).
+template <int L>
+__device__ __forceinline__ float row_sum(float v) {
+  if constexpr (L <= 16) {
+    return group_sum<L>(v);
+  } else {
+    v = group_sum<16>(v);
+    const double r0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
+    const double r1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
+    const double r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
+    const double r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
+    if constexpr (L == 64) return static_cast<float>((r0 + r1) + (r2 + r3));
+    else return static_cast<float>((threadIdx.x & 32) ? r2 + r3 : r0 + r1);
   }
 }
 
@@ -412,28 +430,30 @@ __global__ __launch_bounds__(256) void k_qgemv(QRowsArgs a) {
       }
 #pragma unroll
       for (int r = 0; r < RA; ++r) {
-        float part = 0.0f;
+        float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // four chains: a quarter of the roundings of one
         if constexpr (BITS == 8) {
           qr_h8 p[2];
           qr_unpack8(cur.w[u][r], p);
 #pragma unroll
           for (int q = 0; q < 8; ++q)
-            part = __builtin_amdgcn_fdot2(qr_h2{p[q >> 2][2 * (q & 3)], p[q >> 2][2 * (q & 3) + 1]}, x[q], part, false);
+            ps[q & 3] = __builtin_amdgcn_fdot2(qr_h2{p[q >> 2][2 * (q & 3)], p[q >> 2][2 * (q & 3) + 1]}, x[q],
+                                               ps[q & 3], false);
         } else {
 #pragma unroll
           for (int d = 0; d < 4; ++d) {
             const qr_h8 p = qr_unpack4(cur.w[u][r][d]);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-              part = __builtin_amdgcn_fdot2(qr_h2{p[2 * q], p[2 * q + 1]}, x[4 * d + q], part, false);
+              ps[q] = __builtin_amdgcn_fdot2(qr_h2{p[2 * q], p[2 * q + 1]}, x[4 * d + q], ps[q], false);
           }
         }
+        const float part = (ps[0] + ps[1]) + (ps[2] + ps[3]);
         acc[r] = in ? fmaf(static_cast<float>(cur.s[u][r]), part, acc[r]) : acc[r];
       }
     }
     if (done) {
 #pragma unroll
-      for (int r = 0; r < RA; ++r) acc[r] = group_sum<L>(acc[r]);
+      for (int r = 0; r < RA; ++r) acc[r] = row_sum<L>(acc[r]);
 #pragma unroll
       for (int r = 0; r < RR; ++r) {
         const int n = base + r * RP + sub;
