@@ -325,7 +325,7 @@ int ensure_decode_ws(soc_model* m, int cap) {
   if ((e = hipMemset(w.xcd_ctr, 0, 2 * soc::kXcdGroups * sizeof(int))) != hipSuccess) return hip_fail(e, "hipMemset");
   // step counters of the two one-launch kernels (state[2]: k_decode_persistent, state[3]: k_decode_xcd): each kernel
   // derives its exchange tags from its own count, so the tags of its regions advance by one per layer whichever
-  // decode implementation ran in between
+  // decode implementation ran in between (this copy, on the clears' stream, also waits for them)
   const int32_t step1[2] = {1, 1};
   if ((e = hipMemcpy(w.state + 2, step1, sizeof(step1), hipMemcpyHostToDevice)) != hipSuccess)
     return hip_fail(e, "hipMemcpy");
@@ -373,9 +373,11 @@ int ensure_prefill_ws(soc_model* m, int rows, int total_len, int logit_rows) {
     SOC_TRY(dev_alloc_t(w.allocs, sk, &w.skpart));
     if ((e = soc::skinny_configure()) != hipSuccess) return hip_fail(e, "skinny kernel attributes");
   }
-  if ((e = hipMemset(w.attn_counters, 0, static_cast<size_t>(R) * c.num_key_value_heads * sizeof(int))) != hipSuccess)
+  if ((e = hipMemsetAsync(w.attn_counters, 0, static_cast<size_t>(R) * c.num_key_value_heads * sizeof(int),
+                          m->ctx->stream)) != hipSuccess)
     return hip_fail(e, "hipMemset");
-  if ((e = hipMemset(w.lm_counter, 0, 64 * sizeof(int))) != hipSuccess) return hip_fail(e, "hipMemset");
+  if ((e = hipMemsetAsync(w.lm_counter, 0, 64 * sizeof(int), m->ctx->stream)) != hipSuccess)
+    return hip_fail(e, "hipMemset");
   w.cap_rows = R;
   w.cap_split = SP;
   w.cap_logit_rows = LR;
@@ -975,7 +977,7 @@ int ensure_batch_ws(soc_model* m, int n) {
   SOC_TRY(dev_alloc_t(b.allocs, static_cast<size_t>(n) * soc::kArgmaxMaxChunks, &b.am_val));
   SOC_TRY(dev_alloc_t(b.allocs, static_cast<size_t>(n) * soc::kArgmaxMaxChunks, &b.am_idx));
   SOC_TRY(dev_alloc_t(b.allocs, n, &b.am_cnt));
-  if ((e = hipMemset(b.am_cnt, 0, static_cast<size_t>(n) * sizeof(int32_t))) != hipSuccess)
+  if ((e = hipMemsetAsync(b.am_cnt, 0, static_cast<size_t>(n) * sizeof(int32_t), m->ctx->stream)) != hipSuccess)
     return hip_fail(e, "hipMemset");
   const int columns = std::max({m->qkv_rows, 2 * m->cfg.intermediate_size, m->cfg.hidden_size});
   if (rows) SOC_TRY(dev_alloc_t(b.allocs, soc::gemm_rows_part_floats(n, columns), &b.part));
@@ -2085,7 +2087,7 @@ int run_prefill(soc_model* m, soc_kv* kv, int32_t slot, const int32_t* ids, bool
   record_timer_stop(m->ctx);
   if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "prefill");
   if (id_err != 0) {
-    if ((e = hipMemset(m->ctx->id_err, 0, 4)) != hipSuccess) return hip_fail(e, "hipMemset");
+    if ((e = hipMemsetAsync(m->ctx->id_err, 0, 4, s)) != hipSuccess) return hip_fail(e, "hipMemset");
     return soc::fail(SOC_ERR_INVALID, "token id out of range");
   }
   if (next_token) *next_token = tok;
@@ -2097,7 +2099,7 @@ int ensure_id_flag(soc_ctx* ctx) {
   if (ctx->id_err != nullptr) return SOC_OK;
   hipError_t e = hipMalloc(&ctx->id_err, 64);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc id flag");
-  if ((e = hipMemset(ctx->id_err, 0, 64)) != hipSuccess) return hip_fail(e, "hipMemset");
+  if ((e = hipMemsetAsync(ctx->id_err, 0, 64, ctx->stream)) != hipSuccess) return hip_fail(e, "hipMemset");
   return SOC_OK;
 }
 }  // namespace
@@ -2164,7 +2166,7 @@ int decode_one(soc_model* m, soc_kv* kv, int32_t slot, int32_t last, const int32
   if (trace_path == nullptr) err = rb[1];  // with a trace, run_decode_steps has read the flag itself
   SOC_TRY(one_launch_status(m, xcd, err));
   if (id_err != 0) {
-    if ((e = hipMemset(m->ctx->id_err, 0, 4)) != hipSuccess) return hip_fail(e, "hipMemset");
+    if ((e = hipMemsetAsync(m->ctx->id_err, 0, 4, s)) != hipSuccess) return hip_fail(e, "hipMemset");
     return soc::fail(SOC_ERR_INVALID, "token id out of range");
   }
   kv->len[slot] += 1;
@@ -2524,7 +2526,7 @@ int ensure_op_attention_ws(soc_ctx* ctx, size_t floats, size_t ints) {
     ctx->op_counter_ints = 0;
     if ((e = hipMalloc(&ctx->op_counters, ints * 4)) != hipSuccess) return hip_fail(e, "hipMalloc attention counters");
     // the combining block of each row resets its counter, so the zeros hold from one call to the next
-    if ((e = hipMemset(ctx->op_counters, 0, ints * 4)) != hipSuccess) return hip_fail(e, "hipMemset");
+    if ((e = hipMemsetAsync(ctx->op_counters, 0, ints * 4, ctx->stream)) != hipSuccess) return hip_fail(e, "hipMemset");
     ctx->op_counter_ints = ints;
   }
   return SOC_OK;
@@ -2693,7 +2695,9 @@ int soc_sample_topk(soc_ctx* ctx, const float* row, int32_t vocab, int32_t top_k
       ctx->sample_ws = nullptr;
       ctx->sample_ws_bytes = 0;
       if ((e = hipMalloc(&ctx->sample_ws, need)) != hipSuccess) return hip_fail(e, "hipMalloc sampler workspace");
-      if ((e = hipMemset(ctx->sample_ws, 0, need)) != hipSuccess) {
+      // on the kernels' stream: a clear on the null stream is not ordered with them and could land on what the first
+      // of them has written
+      if ((e = hipMemsetAsync(ctx->sample_ws, 0, need, s)) != hipSuccess) {
         (void)hipFree(ctx->sample_ws);
         ctx->sample_ws = nullptr;
         return hip_fail(e, "hipMemset sampler workspace");

@@ -147,3 +147,19 @@ def test_sample_topk_one_launch_search(gpu_ctx, oracle_mod, k):
                     assert np.array_equal(vals.view(np.uint32), rvals.view(np.uint32))
             finally:
                 gpu_ctx.free(p)
+
+
+def test_sample_topk_on_a_new_workspace(gpu_ctx):
+    """The first call of a context clears its workspace and searches in it at once: the clear comes before the search's
+    writes (on another stream it could land between them and lose candidates)."""
+    row = np.random.default_rng(5).standard_normal(400000).astype(np.float32)
+    want = np.argsort(-row, kind="stable")[:5]
+    for _ in range(12):
+        ctx = S.Context(0)
+        p = ctx.upload(row)
+        try:
+            _, ids, _ = S.sample_topk(ctx, p, row.size, 5, 1.0)
+            np.testing.assert_array_equal(ids, want)
+        finally:
+            ctx.free(p)
+            ctx.close()
