@@ -362,18 +362,27 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int qpos, Att
   }
   __syncthreads();
   // a wave per head, a lane per chunk (one thread walking 64 chunks' maxima and exponentials took as long as the
-  // chunk itself)
+  // chunk itself); the sums in chunk order, from LDS
   for (int j = wid; j < G; j += 4) {
     float M = -INFINITY;
     for (int t = lane; t < nact; t += 64) M = fmaxf(M, cm[j][t]);
     M = wave_max(M);
+    for (int t = lane; t < nact; t += 64) cm[j][t] = expf(cm[j][t] - M);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the sums read the other lanes' weights
+    __builtin_amdgcn_wave_barrier();
     float L = 0.0f;
-    for (int t = lane; t < nact; t += 64) {
-      const float e = expf(cm[j][t] - M);
-      cm[j][t] = e;
-      L += cl[j][t] * e;
+    for (int t0 = 0; t0 < nact; t0 += 8) {
+      float e[8], l[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int t = min(t0 + u, nact - 1);
+        e[u] = cm[j][t];
+        l[u] = cl[j][t];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (t0 + u < nact) L = fmaf(l[u], e[u], L);
     }
-    L = wave_sum(L);
     if (lane == 0) lstat[j] = L;
   }
   __syncthreads();

@@ -290,7 +290,8 @@ k_qrows(QRowsArgs a) {
   }
 }
 
-// group_sum<L> with the sums of 16 lanes added in float64 (two to four terms: one rounding instead of up to two levels).
+// group_sum<L> with the sums of 16 lanes added in float64 (two to four terms: one rounding instead of up to two levels),
+// for soc_qmm.
 template <int L>
 __device__ __forceinline__ float row_sum(float v) {
   if constexpr (L <= 16) {
@@ -311,14 +312,20 @@ __device__ __forceinline__ float row_sum(float v) {
 // (v_dot2_f32_f16 on the unpacked pairs; 16 rows of 64 bytes per load, as the matrix cores want them, stream more
 // slowly). RR rows per lane group are in flight at once, U chunks of each; the first are requested before the
 // activations are staged (fp16 in the codes' order, in LDS). SwiGLU: RR gate rows and their up rows.
+//
+// Inside a model's layers the sums keep the order of the separate kernels (k_qmm, k_rmsnorm_rows_v) that these forms
+// fused: a chunk's products in one chain, a row's lanes by group_sum, the squares of RMSNorm by one wave. Every
+// projection rounds its input to fp16, so another order of fp32 sums flips roundings that travel through the layers
+// (3e-4 to 6e-4 of the logits over four layers, as far from 64 bits on average: 6.9e-4 and 7.0e-4). soc_qmm (QX_F16,
+// EPI_STORE), whose sums are its result, takes four chains and row_sum.
 template <int BITS, int L, int RR, int U, int XF, int EPI>
 __global__ __launch_bounds__(256) void k_qgemv(QRowsArgs a) {
   extern __shared__ __attribute__((aligned(16))) u32x4 qx[];  // [K / 8]
-  __shared__ float ssw[4];
   constexpr int CH = BITS == 8 ? 16 : 32;         // codes per 16-byte chunk
   constexpr int RP = 64 / L;                      // lane groups
   constexpr bool AHEAD = RR == 1;                 // (tall matrices: more waves resident instead)
   constexpr int RA = EPI == EPI_SWIGLU ? 2 * RR : RR;
+  constexpr bool QMM = XF == QX_F16 && EPI == EPI_STORE;
   const int tid = threadIdx.x, lane = tid & 63, sub = lane / L, ln = lane % L;
   const int K = a.K, nch = K / CH, G = K / 64;
   const int nout = EPI == EPI_SWIGLU ? a.N / 2 : a.N;
@@ -358,29 +365,35 @@ __global__ __launch_bounds__(256) void k_qgemv(QRowsArgs a) {
     }
   };
   if constexpr (XF == QX_NORM) {
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u) values(min(tid + 256 * u, K / 8 - 1), keep[u]);
+    // every wave sums the whole row's squares (a few KB of L1), four loads in flight: no barrier
     float ss = 0.0f;
+    const int nv = K / 4;
+    for (int i0 = lane; i0 < nv; i0 += 4 * 64) {
+      f32x4 v[4];
 #pragma unroll
-    for (int u = 0; u < KEEP; ++u) {
-      values(min(tid + 256 * u, K / 8 - 1), keep[u]);
-      if (tid + 256 * u < K / 8)
+      for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const f32x4*>(a.x + 4 * min(i0 + 64 * u, nv - 1));
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ss = fmaf(keep[u][e], keep[u][e], ss);
+      for (int u = 0; u < 4; ++u)
+        if (i0 + 64 * u < nv) {
+          ss = i0 + u == lane ? fmaf(v[u][0], v[u][0], v[u][1] * v[u][1])
+                              : fmaf(v[u][1], v[u][1], fmaf(v[u][0], v[u][0], ss));
+          ss = fmaf(v[u][3], v[u][3], fmaf(v[u][2], v[u][2], ss));
+        }
     }
-    for (int i = tid + 256 * KEEP; i < K / 8; i += 256) {
-      float f[8];
-      values(i, f);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
-    }
-    ss = block_sum<256>(ss, ssw);
-    rs = 1.0f / sqrtf(ss / static_cast<float>(K) + a.eps);
+    rs = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(K) + a.eps);
   }
   auto stage = [&](int i, const float (&f)[8]) {
     f16x8 v;
     if constexpr (XF == QX_NORM) {
       const f16x8 gn = as_f16x8(load16(a.gain + 8 * i));
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = static_cast<f16>(f[e] * rs * static_cast<float>(gn[e]));
+      for (int e = 0; e < 8; ++e) {
+        float y = f[e] * rs * static_cast<float>(gn[e]);
+        __asm__ volatile("" : "+v"(y));  // rounded to fp32, then to fp16 (v_fma_mixlo_f16 would round once)
+        v[e] = static_cast<f16>(y);
+      }
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = static_cast<f16>(f[e]);
@@ -430,30 +443,34 @@ __global__ __launch_bounds__(256) void k_qgemv(QRowsArgs a) {
       }
 #pragma unroll
       for (int r = 0; r < RA; ++r) {
-        float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // four chains: a quarter of the roundings of one
+        constexpr int NC = QMM ? 4 : 1;  // chains: of four, each has a quarter of the roundings
+        float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         if constexpr (BITS == 8) {
           qr_h8 p[2];
           qr_unpack8(cur.w[u][r], p);
 #pragma unroll
           for (int q = 0; q < 8; ++q)
-            ps[q & 3] = __builtin_amdgcn_fdot2(qr_h2{p[q >> 2][2 * (q & 3)], p[q >> 2][2 * (q & 3) + 1]}, x[q],
-                                               ps[q & 3], false);
+            ps[q % NC] = __builtin_amdgcn_fdot2(qr_h2{p[q >> 2][2 * (q & 3)], p[q >> 2][2 * (q & 3) + 1]}, x[q],
+                                                ps[q % NC], false);
         } else {
 #pragma unroll
           for (int d = 0; d < 4; ++d) {
             const qr_h8 p = qr_unpack4(cur.w[u][r][d]);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-              ps[q] = __builtin_amdgcn_fdot2(qr_h2{p[2 * q], p[2 * q + 1]}, x[4 * d + q], ps[q], false);
+              ps[q % NC] = __builtin_amdgcn_fdot2(qr_h2{p[2 * q], p[2 * q + 1]}, x[4 * d + q], ps[q % NC], false);
           }
         }
-        const float part = (ps[0] + ps[1]) + (ps[2] + ps[3]);
+        const float part = QMM ? (ps[0] + ps[1]) + (ps[2] + ps[3]) : ps[0];
         acc[r] = in ? fmaf(static_cast<float>(cur.s[u][r]), part, acc[r]) : acc[r];
       }
     }
     if (done) {
 #pragma unroll
-      for (int r = 0; r < RA; ++r) acc[r] = row_sum<L>(acc[r]);
+      for (int r = 0; r < RA; ++r) {
+        if constexpr (QMM) acc[r] = row_sum<L>(acc[r]);
+        else acc[r] = group_sum<L>(acc[r]);
+      }
 #pragma unroll
       for (int r = 0; r < RR; ++r) {
         const int n = base + r * RP + sub;

@@ -91,3 +91,24 @@ def test_quantized_layer_widths(gpu_ctx, oracle_mod, bits, hidden, inter, n):
     finally:
         kv.close()
         m.close()
+
+
+@pytest.mark.parametrize("length", [97, 300])
+@pytest.mark.parametrize("bits", [8, 4])
+def test_quantized_decode_keeps_its_bits(gpu_ctx, golden, bits, length):
+    """One decode row of a quantized model in the summation order of separate norm, projection, SwiGLU and residual
+    kernels, bit for bit: tests/golden/qdecode_rows.npz holds the logits of four steps that those kernels gave
+    (Qwen3-0.6B widths, two layers, 97 and 300 cached keys: one attention chunk and five). Every projection rounds its
+    input to fp16, so any other order shows as a few 1e-4."""
+    cfg = S.QwenConfig(vocab_size=256, hidden_size=1024, num_hidden_layers=2, num_attention_heads=16,
+                       num_key_value_heads=8, intermediate_size=3072)
+    m = S.Model(gpu_ctx, cfg).load(S.synth_weights(cfg, 81)).quantize(bits)
+    kv = S.KVCache(m, 1, 320)
+    try:
+        kv.fill_synthetic(0, length, 82)
+        got = np.stack([S.decode(m, kv, 0, t)[0] for t in (11, 200, 77, 5)])
+    finally:
+        kv.close()
+        m.close()
+    want = golden("qdecode_rows.npz")[f"int{bits}_{length}"]
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), float(np.max(np.abs(got - want)))
