@@ -189,10 +189,12 @@ bool sample_device_fits(int V, int k);
 // Device workspace bytes for a row of V logits; zero-filled when allocated (its first word is an arrival counter
 // that every launch_sample_head leaves at zero).
 size_t sample_ws_bytes(int V);
-// The search in one launch, for rows whose k largest values of row / t differ (and any row at k = 1): out[0] = k,
-// out[1] = 0, then k (index, bits of its raw logit) pairs from the largest down. out[1] = 1: the row holds a NaN;
-// out[1] = 2: equal values among the k largest, launch_sample_topk has to search. out takes 2 + 2 k words, in device or
+// The search in one launch: out[0] = count, out[1] = 0, then count (index, bits of its raw logit) pairs: the k largest
+// values of row / t from the largest down where they differ (and at k = 1), else candidates in index order, all that
+// std::partial_sort(top k of row / t) moves into its heap among them. out[1] = 1: the row holds a NaN; out[1] = 2: more
+// candidates than kSampleHeadMax, launch_sample_topk has to search. out takes 2 + 2 kSampleHeadMax words, in device or
 // pinned host memory. Requires sample_head_fits(V, k).
+constexpr int kSampleHeadMax = 2048;
 bool sample_head_fits(int V, int k);
 hipError_t launch_sample_head(const float* row, int V, float t, int k, void* ws, int* out, hipStream_t s);
 // Finds the candidates that std::partial_sort(top k of row / t) over 0..V-1 moves into its heap, in index order:

@@ -2705,6 +2705,7 @@ int soc_sample_topk(soc_ctx* ctx, const float* row, int32_t vocab, int32_t top_k
       ctx->sample_ws_bytes = need;
     }
     constexpr size_t kOutInts = 2 + 2 * static_cast<size_t>(kMaxOut);
+    static_assert(soc::kSampleHeadMax <= kMaxOut, "output block");
     if (ctx->sample_out == nullptr && (e = hipMalloc(&ctx->sample_out, kOutInts * sizeof(int))) != hipSuccess)
       return hip_fail(e, "hipMalloc sampler output");
     if (ctx->sample_host == nullptr &&
@@ -2715,7 +2716,7 @@ int soc_sample_topk(soc_ctx* ctx, const float* row, int32_t vocab, int32_t top_k
             hipSuccess)
       return hip_fail(e, "hipHostGetDevicePointer");
     // one launch that writes its candidates into pinned host memory; the general search and its copies only for a row
-    // with equal values among its k largest
+    // of equal values among its k largest and many candidates (rising rows)
     const int* out = ctx->sample_host;
     int n = 0, flag = 2;
     if (soc::sample_head_fits(vocab, k)) {

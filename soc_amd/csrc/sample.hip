@@ -23,9 +23,12 @@
 // which k_topk_one finds in one launch.
 //
 // Where the k largest q differ from each other and from the rest, the heap's history does not matter: any sort returns
-// those k in descending order. k_topk_distinct finds them in one launch and says when they do not differ; only then
-// do the three kernels above run.
+// those k in descending order. k_topk_head finds them in one launch, and where they do not differ a superset of S in
+// index order (candidates that do not enter are not touched, so any superset serves). Only where that grows past what
+// one block ranks (rising rows) do the three kernels above run.
 #include "kernels.h"
+
+#include <type_traits>
 
 namespace soc {
 namespace {
@@ -392,21 +395,34 @@ __global__ __launch_bounds__(NT) void k_topk_one(const float* __restrict__ row, 
   }
 }
 
-// ---- the k largest values of a row whose top k differ, in one launch -------------------------------------------
+// ---- the candidates of a row in one launch ----------------------------------------------------------------------
 // Bound by latency, not by the 4 V bytes: a load round trip, the arrival counter, and a chain of short steps in the
 // last block to arrive. The row is cut into groups of FE << gshift values (the lanes of a wave that share the tid's
 // upper bits); every block publishes its groups' maxima. With T any value that at least k group maxima reach, the k
-// largest values are all >= T and lie in the groups whose maximum is, so the last block raises T bit by bit until few
+// largest values are all >= T and lie in the groups whose maximum is, so the last block halves towards T until few
 // more than k groups are left (4 V bytes are never sorted; no repeated extraction of maxima), reads those groups
 // again, and ranks the values >= T among themselves. Top 50 of 151936 at temperature 0.7, MI355X: 107 us of kernels
-// for the general search (74 of them the prefix walk of the last chunk) against 17.5 us, 121 -> 30 us for the call.
+// for the general search (74 of them the prefix walk of the last chunk) against 17.5 us, 121 -> 29 us for the call.
+//
+// Equal values among the k largest (the rule for logits that were rounded to 16 bits) make the heap's history matter.
+// The same block then bounds the heap's root from below at doubling prefixes of the row: 128 .. 2048 values of the
+// first chunk, 2 .. 64 chunks of group maxima, one wave's search each. A value that enters is above the bound of
+// the last such prefix before it, so the first 128 values and the values above their bound, about k per doubling,
+// hold S. us a call at 50 of 151936 / 50 of 4096 / 20 of 32000, this kernel followed by the general search, that search
+// alone, this: rounded to bf16 149 / 113 / 88, 121 / 90 / 63, 78 / 49 / 46; all but 20 masked 149 / 105 / 78, 118 / 75 /
+// 47, 34 / 34 / 35. Two of 32000 that are equal 60, 36, 43. Rows that rise end to end overflow and take both: 258 at 50
+// of 4096, 220 for the general search alone.
 constexpr int FT = 512;                 // threads per block
+constexpr int FW = FT / kWave;
 constexpr int FE = kSampleChunk / FT;   // values per thread
 constexpr int FR = 16;                  // group maxima per thread of the last block
 constexpr int kMaxGroups = FR * FT;
-constexpr int kMaxSel = 512;            // groups read again
-constexpr int kMaxCand = 1088;          // values ranked
+constexpr int kMaxSel = 1024;           // groups read again
+constexpr int kMaxRank = 1088;          // values ranked by value
+constexpr int kMaxCand = kSampleHeadMax;  // values ranked by index
 constexpr int kSlack = 32;              // groups beyond k that end the search for T
+constexpr int kPrefixes = 11;           // bounds: prefixes of 128 << b values (b < 5), of 2 << (b - 5) chunks
+constexpr int kPrefixRegs = 32;         // keys per lane of a prefix search
 
 // Values in ascending order of q as unsigned words, equal q (+0 and -0 too) as equal words, all above 0; 0 stands for
 // no value.
@@ -415,16 +431,89 @@ __device__ __forceinline__ uint32_t key_of(float q) {
   return (b & 0x80000000u) ? ~b : b | 0x80000000u;
 }
 
-// out[1]: 0 = out[0] = k entries follow in descending order (index, bits of the raw logit); 1 = the row holds a NaN;
-// 2 = equal values among the k largest, or too many values near them.
-__global__ __launch_bounds__(FT) void k_topk_distinct(const float* __restrict__ row, int V, float t, int k, int gshift,
-                                                       int32_t* __restrict__ gmax, int32_t* __restrict__ gnan,
-                                                       int* __restrict__ counter, int* __restrict__ out) {
+// Minimum and maximum over the wave (DPP within rows of 16 lanes, then the four rows).
+template <bool MIN>
+__device__ __forceinline__ uint32_t wave_pick(uint32_t v) {
+  auto pick = [](uint32_t a, uint32_t b) { return MIN ? min(a, b) : max(a, b); };
+  auto mov = [](uint32_t a, auto ctrl) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(a), decltype(ctrl)::value, 0xF, 0xF, true));
+  };
+  v = pick(v, mov(v, std::integral_constant<int, 0xB1>()));
+  v = pick(v, mov(v, std::integral_constant<int, 0x4E>()));
+  v = pick(v, mov(v, std::integral_constant<int, 0x141>()));
+  v = pick(v, mov(v, std::integral_constant<int, 0x140>()));
+  const uint32_t a = __builtin_amdgcn_readlane(v, 0), b = __builtin_amdgcn_readlane(v, 16),
+                 c = __builtin_amdgcn_readlane(v, 32), d = __builtin_amdgcn_readlane(v, 48);
+  return pick(pick(a, b), pick(c, d));
+}
+
+// The wave's keys (N per lane, those from `regs` on absent) against a pivot: how many reach it, the smallest that does
+// (all ones: none) and the largest that does not.
+struct Split {
+  int n;
+  uint32_t least, below;
+};
+template <int N>
+__device__ __forceinline__ Split wave_split(const uint32_t (&key)[N], int regs, uint32_t pivot) {
+  Split r{0, 0xFFFFFFFFu, 0u};
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+    if (u < regs) {
+      const bool in = key[u] >= pivot;
+      r.n += __popcll(__ballot(in));
+      r.least = min(r.least, in ? key[u] : 0xFFFFFFFFu);
+      r.below = max(r.below, in ? 0u : key[u]);
+    }
+  r.least = wave_pick<true>(r.least);
+  r.below = wave_pick<false>(r.below);
+  return r;
+}
+
+// Where a search starts: how many keys there are (0: none), the smallest and the largest.
+template <int N>
+__device__ __forceinline__ Split wave_range(const uint32_t (&key)[N], int regs) {
+  Split r{0, 0xFFFFFFFFu, 0u};
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+    if (u < regs) {
+      r.n += __popcll(__ballot(key[u] != 0));
+      r.least = min(r.least, key[u] - 1);  // (0 becomes all ones)
+      r.below = max(r.below, key[u]);
+    }
+  r.least = wave_pick<true>(r.least) + 1;
+  r.below = wave_pick<false>(r.below);
+  return r;
+}
+
+// A search for a key that at least k keys reach and few more than k do, by halving [lo, hi): n keys reach lo, fewer
+// than k reach hi. Both ends move on to a key that is there, so equal keys end it in a step or two (bit by bit they
+// took all 32).
+struct Search {
+  uint32_t lo, hi;
+  int n;
+  __device__ __forceinline__ bool done(int enough) const { return n <= enough || hi - lo <= 1; }
+  __device__ __forceinline__ uint32_t pivot() const { return lo + (hi - lo) / 2; }
+  __device__ __forceinline__ void step(const Split& s, int k) {
+    if (s.n >= k) {
+      lo = s.least;
+      n = s.n;
+    } else {
+      hi = s.below + 1;
+    }
+  }
+};
+
+// out[1]: 0 = out[0] entries follow: either the k largest in descending order or candidates in index order (index, bits
+// of the raw logit); 1 = the row holds a NaN; 2 = too many candidates.
+__global__ __launch_bounds__(FT) void k_topk_head(const float* __restrict__ row, int V, float t, int k, int gshift,
+                                                   int32_t* __restrict__ gmax, int32_t* __restrict__ gnan,
+                                                   int* __restrict__ counter, int* __restrict__ out) {
   __shared__ int sel[kMaxSel];
-  __shared__ uint32_t ckey[kMaxCand];
+  __shared__ uint32_t ckey[kMaxRank];
   __shared__ int cidx[kMaxCand];
   __shared__ float craw[kMaxCand];
-  __shared__ int wsum[2][FT / kWave];
+  __shared__ uint32_t bound[kPrefixes];
+  __shared__ Split part[2][FW];
   __shared__ int nsel, ncand, last;
   const int c = blockIdx.x, nch = gridDim.x, tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
   const int gpb = FT >> gshift;  // groups per block
@@ -468,24 +557,30 @@ __global__ __launch_bounds__(FT) void k_topk_distinct(const float* __restrict__ 
     }
     return;
   }
-  uint32_t T = 0;
-  for (int bit = 31; bit >= 0; --bit) {
-    const uint32_t trial = T | (1u << bit);
-    int n = 0;
-#pragma unroll
-    for (int u = 0; u < FR; ++u)
-      if (u * FT < G) n += __popcll(__ballot(g[u] >= trial));
-    if (lane == 0) wsum[bit & 1][w] = n;
+  // T among all group maxima, one barrier a step
+  const int regs = (G + FT - 1) / FT;
+  auto block_merge = [&](const Split& p, int buf) {
+    if (lane == 0) part[buf][w] = p;
     __syncthreads();
-    n = 0;
+    Split r = part[buf][0];
 #pragma unroll
-    for (int u = 0; u < FT / kWave; ++u) n += wsum[bit & 1][u];
-    if (n >= k) {
-      T = trial;
-      if (n <= k + kSlack) break;
+    for (int u = 1; u < FW; ++u) {
+      const Split o = part[buf][u];
+      r.n += o.n;
+      r.least = min(r.least, o.least);
+      r.below = max(r.below, o.below);
     }
+    return r;
+  };
+  uint32_t T = 1;  // fewer than k groups: every value
+  Split p = wave_range(g, regs);
+  if (p.n == 0) p.least = 0xFFFFFFFFu;
+  const Split all = block_merge(p, 1);
+  if (all.n >= k) {
+    Search f{all.least, all.below + 1, all.n};
+    for (int buf = 0; !f.done(k + kSlack); buf ^= 1) f.step(block_merge(wave_split(g, regs, f.pivot()), buf), k);
+    T = f.lo;
   }
-  T = max(T, 1u);  // fewer than k groups: every value
 #pragma unroll
   for (int u = 0; u < FR; ++u)
     if (g[u] >= T) {
@@ -493,63 +588,161 @@ __global__ __launch_bounds__(FT) void k_topk_distinct(const float* __restrict__ 
       if (p < kMaxSel) sel[p] = u * FT + tid;
     }
   __syncthreads();
-  const int ns = nsel;
-  bool give_up = ns > kMaxSel;
   const int gs = gshift + 2;  // log2 of the values per group
   static_assert(FE == 4, "values per group");
-  for (int p0 = 0; !give_up && p0 < (ns << gs); p0 += 8 * FT) {
-    int ix[8];
-    float y[8];
+  // hands every value of the ns selected groups to take(group, index, raw)
+  auto read_groups = [&](int ns, auto take) {
+    for (int p0 = 0; p0 < (ns << gs); p0 += 8 * FT) {
+      int gr[8], ix[8];
+      float y[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int p = p0 + u * FT + tid;
-      ix[u] = V;
-      if (p < (ns << gs)) {
-        const int gi = sel[p >> gs], j = p & ((1 << gs) - 1);
-        ix[u] = (gi / gpb) * kSampleChunk + (j >> gshift) * FT + ((gi % gpb) << gshift) + (j & ((1 << gshift) - 1));
-      }
-      y[u] = row[min(ix[u], V - 1)];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const uint32_t key = key_of(__fdiv_rn(y[u], t));
-      if (ix[u] < V && key >= T) {
-        const int r = atomicAdd(&ncand, 1);
-        if (r < kMaxCand) {
-          ckey[r] = key;
-          cidx[r] = ix[u];
-          craw[r] = y[u];
+      for (int u = 0; u < 8; ++u) {
+        const int p = p0 + u * FT + tid;
+        gr[u] = 0;
+        ix[u] = V;
+        if (p < (ns << gs)) {
+          const int gi = gr[u] = sel[p >> gs], j = p & ((1 << gs) - 1);
+          ix[u] = (gi / gpb) * kSampleChunk + (j >> gshift) * FT + ((gi % gpb) << gshift) + (j & ((1 << gshift) - 1));
         }
+        y[u] = row[min(ix[u], V - 1)];
       }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (ix[u] < V) take(gr[u], ix[u], y[u]);
+    }
+  };
+  bool give_up = nsel > kMaxSel / 2;
+  if (!give_up)
+    read_groups(nsel, [&](int, int i, float y) {
+      const uint32_t key = key_of(__fdiv_rn(y, t));
+      if (key < T) return;
+      const int r = atomicAdd(&ncand, 1);
+      if (r < kMaxRank) {
+        ckey[r] = key;
+        cidx[r] = i;
+        craw[r] = y;
+      }
+    });
+  __syncthreads();
+  int n = ncand;
+  give_up |= n > kMaxRank;
+  constexpr int RK = (kMaxRank + FT - 1) / FT;
+  int rank[RK];
+  if (!give_up) {
+#pragma unroll
+    for (int u = 0; u < RK; ++u) {
+      rank[u] = k;
+      const int i = tid + u * FT;
+      if (i >= n) continue;
+      const uint32_t key = ckey[i];
+      int above = 0, same = 0;
+#pragma unroll 8
+      for (int j = 0; j < n; ++j) {
+        above += ckey[j] > key;
+        same += ckey[j] == key;
+      }
+      rank[u] = above;
+      give_up |= above < k && same > 1;
+    }
+  }
+  if (!__syncthreads_or(give_up)) {
+#pragma unroll
+    for (int u = 0; u < RK; ++u)
+      if (rank[u] < k) {
+        out[2 + 2 * rank[u]] = cidx[tid + u * FT];
+        out[3 + 2 * rank[u]] = __float_as_int(craw[tid + u * FT]);
+      }
+    if (tid == 0) {
+      out[0] = k;
+      out[1] = 0;
+    }
+    return;
+  }
+
+  // Equal values (or many near the k-th): bounds of the heap's root by prefix, a wave each, the long ones in waves of
+  // one task. A prefix that does not end before the row's last value bounds nothing.
+  if (tid == 0) nsel = ncand = 0;
+  for (int task = w; task < kPrefixes; task += FW) {
+    // a digit per task, from the right: 128, 256 values, 2 chunks | 2048 values, 64 chunks, 1024 values, 32, 16 chunks |
+    // 512 values, 4, 8 chunks
+    const int b = static_cast<int>(0x762893A4510ull >> 4 * task) & 15;
+    const bool vals = b < 5;
+    const int len = vals ? 128 << b : 2 << (b - 5);  // values, or chunks
+    uint32_t B = 0;
+    if (vals ? len < V : len < nch) {
+      const int cnt = vals ? len : min(len * gpb, kPrefixRegs * kWave);  // (of a part of the prefix: a lower bound too)
+      uint32_t key[kPrefixRegs];
+#pragma unroll
+      for (int u = 0; u < kPrefixRegs; ++u) {
+        key[u] = 0;
+        const int i = u * kWave + lane;
+        if (u * kWave < cnt && i < cnt)
+          key[u] = vals ? key_of(__fdiv_rn(row[i], t)) : static_cast<uint32_t>(ld_dev(gmax + i));
+      }
+      const int held = (cnt + kWave - 1) / kWave;
+      const Split all = wave_range(key, held);
+      Search f{all.least, all.below + 1, all.n};
+      while (!f.done(max(k + k / 8, kSlack))) f.step(wave_split(key, held, f.pivot()), k);
+      B = f.lo;
+    }
+    if (lane == 0) bound[b] = B;
+  }
+  __syncthreads();
+  auto chunk_bound = [&](int ch) {  // chunks from 1
+    return ch == 1 ? bound[4] : bound[5 + min(31 - __clz(ch), 6) - 1];
+  };
+  auto put = [&](int i, float y, uint32_t key, uint32_t b) {
+    if (key <= b) return;
+    const int r = atomicAdd(&ncand, 1);
+    if (r < kMaxCand) {
+      cidx[r] = i;
+      craw[r] = y;
+    }
+  };
+#pragma unroll
+  for (int e = 0; e < FE; ++e) {  // the first chunk
+    const int i = e * FT + tid;
+    if (i < min(V, kSampleChunk)) {
+      const float y = row[i];
+      put(i, y, key_of(__fdiv_rn(y, t)), i < 128 ? 0u : bound[31 - __clz(i) - 7]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < FR; ++u) {
+    const int gi = u * FT + tid;
+    if (gi < G && gi >= gpb && g[u] > chunk_bound(gi / gpb)) {
+      const int p = atomicAdd(&nsel, 1);
+      if (p < kMaxSel) sel[p] = gi;
     }
   }
   __syncthreads();
-  const int n = ncand;
-  give_up |= n > kMaxCand;
-  if (!give_up) {
-    for (int i = tid; i < n; i += FT) {
-      const uint32_t key = ckey[i];
-      int rank = 0, same = 0;
-#pragma unroll 8
-      for (int j = 0; j < n; ++j) {
-        rank += ckey[j] > key;
-        same += ckey[j] == key;
-      }
-      if (rank < k) {
-        give_up |= same > 1;
-        out[2 + 2 * rank] = cidx[i];
-        out[3 + 2 * rank] = __float_as_int(craw[i]);
-      }
+  const int ns = nsel;
+  if (ns <= kMaxSel)
+    read_groups(ns, [&](int gi, int i, float y) { put(i, y, key_of(__fdiv_rn(y, t)), chunk_bound(gi / gpb)); });
+  __syncthreads();
+  n = ncand;
+  if (ns > kMaxSel || n > kMaxCand) {
+    if (tid == 0) {
+      out[0] = 0;
+      out[1] = 2;
     }
+    return;
   }
-  const int any = __syncthreads_or(give_up);
+  for (int i = tid; i < n; i += FT) {
+    const int at = cidx[i];
+    int r = 0;
+#pragma unroll 8
+    for (int j = 0; j < n; ++j) r += cidx[j] < at;
+    out[2 + 2 * r] = at;
+    out[3 + 2 * r] = __float_as_int(craw[i]);
+  }
   if (tid == 0) {
-    out[0] = k;
-    out[1] = any ? 2 : 0;
+    out[0] = n;
+    out[1] = 0;
   }
 }
 
-// Lanes per group (log2) of k_topk_distinct: groups of 64 values, or 16 where a row of 64-value groups would have few
+// Lanes per group (log2) of k_topk_head: groups of 64 values, or 16 where a row of 64-value groups would have few
 // more of them than k.
 int distinct_gshift(int V) { return V >= 32768 ? 4 : 2; }
 
@@ -572,7 +765,7 @@ hipError_t launch_sample_head(const float* row, int V, float t, int k, void* ws,
   if (k == 1)  // partials in the first entries of the lists' regions
     hipLaunchKernelGGL(k_topk_one, dim3(nch), dim3(NT), 0, s, row, V, t, chunk_top, acc_cnt, chunk_nan, counter, out);
   else  // the group maxima (at most 128 of a chunk's 2048 values) in the entrants' region
-    hipLaunchKernelGGL(k_topk_distinct, dim3(nch), dim3(FT), 0, s, row, V, t, k, distinct_gshift(V), acc_idx, chunk_nan,
+    hipLaunchKernelGGL(k_topk_head, dim3(nch), dim3(FT), 0, s, row, V, t, k, distinct_gshift(V), acc_idx, chunk_nan,
                        counter, out);
   return hipGetLastError();
 }

@@ -163,3 +163,32 @@ def test_sample_topk_on_a_new_workspace(gpu_ctx):
         finally:
             ctx.free(p)
             ctx.close()
+
+
+@pytest.mark.parametrize("k", [2, 20, 50, 64])
+def test_sample_topk_equal_values_in_one_launch(gpu_ctx, oracle_mod, k):
+    """Rows with equal values among their k largest, where the order of the result follows the history of the
+    reference's heap: at the edges of the prefixes that bound it (128 .. 2048 values of the first chunk, 2 .. 64 chunks,
+    groups of 16 and of 64 values), logits rounded to 16 bits, small integers, one value alone, all but a few masked
+    with -inf or the type's lowest value, and rising and falling rows (rising ones overflow the one launch into the
+    general search). Bit for bit the oracle's candidates."""
+    rng = np.random.default_rng(100 + k)
+    lowest = np.finfo(np.float32).min
+    for v in (127, 128, 129, 255, 257, 1025, 2047, 2049, 4097, 8193, 32767, 32768, 65 * 2048 + 1, 151936, 262145):
+        normal = rng.standard_normal(v) * 2
+        masked = np.full(v, -np.inf)
+        masked[rng.integers(0, v, 9)] = rng.integers(0, 3, 9)
+        rows = {"fp16": normal.astype(np.float16), "fewer bits": np.round(normal * 4) / 4,
+                "one value": np.full(v, -0.0), "-inf": masked, "lowest": np.maximum(masked, lowest),
+                "rising": np.sort(normal.astype(np.float16)), "falling": np.sort(normal.astype(np.float16))[::-1]}
+        for what, row in rows.items():
+            r = np.ascontiguousarray(row, np.float32)
+            p = gpu_ctx.upload(r)
+            try:
+                for t in (1.0, 0.7):
+                    tok, ids, vals = S.sample_topk(gpu_ctx, p, v, k, t)
+                    rtok, rids, rvals = oracle_mod.sample_topk(r, t, k)
+                    assert tok == rtok and np.array_equal(ids, rids), f"{what}, V {v}, temperature {t}"
+                    assert np.array_equal(vals.view(np.uint32), rvals.view(np.uint32)), f"{what}, V {v}"
+            finally:
+                gpu_ctx.free(p)
