@@ -35,8 +35,8 @@ struct soc_ctx {
   int* sample_out = nullptr;
   int* sample_host = nullptr;   // pinned host copy of the output block (hipHostMalloc)
   int* sample_host_dev = nullptr;  // the address kernels use for it
-  // pinned host words a decode step's readback kernel writes (next token, wait error, token id error), with the
-  // address kernels use for them
+  // pinned host words a decode step's readback kernel writes (next token, wait error, token id error), then a batch's
+  // ids, slots and positions on their way in and tokens on their way out, with the address kernels use for them
   int32_t* readback = nullptr;
   int32_t* readback_dev = nullptr;
   // op-level attention (soc_attention_decode): split-key partials and arrival counters, grown on demand

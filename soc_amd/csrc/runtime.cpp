@@ -116,9 +116,6 @@ struct PrefillWs {
 struct BatchWs {
   int cap = 0;
   int32_t *ids = nullptr, *pos = nullptr, *start = nullptr, *slots = nullptr;
-  // pinned: a call's ids, slots and positions (n each) on their way in, then at 3 cap soc_decode_batch's tokens on
-  // their way out; host_dev is the address kernels use
-  int32_t *host = nullptr, *host_dev = nullptr;
   // per-row candidates and arrival counters of the split greedy argmax ([cap][kArgmaxMaxChunks], [cap])
   float* am_val = nullptr;
   int32_t *am_idx = nullptr, *am_cnt = nullptr;
@@ -948,6 +945,21 @@ int validate_ids(const soc_model* m, const int32_t* ids, int n) {
 }
 
 
+// The context's pinned words (soc_ctx::readback), allocated on first use.
+constexpr size_t kReadbackBatch = 16;  // where a batch's rows begin
+int ensure_readback(soc_ctx* ctx) {
+  if (ctx->readback != nullptr) return SOC_OK;
+  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&ctx->readback),
+                               (kReadbackBatch + static_cast<size_t>(4) * kMaxBatchRows) * sizeof(int32_t));
+  if (e != hipSuccess) return hip_fail(e, "hipHostMalloc readback words");
+  if ((e = hipHostGetDevicePointer(reinterpret_cast<void**>(&ctx->readback_dev), ctx->readback, 0)) != hipSuccess) {
+    (void)hipHostFree(ctx->readback);
+    ctx->readback = nullptr;
+    return hip_fail(e, "hipHostGetDevicePointer");
+  }
+  return SOC_OK;
+}
+
 // A batch step's projections: the skinny kernels (input RMSNorm, q/k norm, RoPE and KV append folded in) up to their 16
 // rows, else the split-K row GEMMs, which stream the weights once whatever the rows (two layers and a 16384-word head,
 // us per step, against skinny slabs of 16: Qwen3-0.6B 17 rows 198 : 277, 64 rows 226 : 470; Qwen3-4B 17 rows 329 : 400,
@@ -955,6 +967,7 @@ int validate_ids(const soc_model* m, const int32_t* ids, int n) {
 bool batch_skinny_path(const soc_model* m, int n) { return m->pws.skpart != nullptr && n <= 16; }
 
 int ensure_batch_ws(soc_model* m, int n) {
+  SOC_TRY(ensure_readback(m->ctx));
   BatchWs& b = m->bws;
   const bool rows = !batch_skinny_path(m, n);  // needs the row GEMMs' partial sums
   if (b.cap >= n && (b.part != nullptr || !rows)) return SOC_OK;
@@ -962,14 +975,8 @@ int ensure_batch_ws(soc_model* m, int n) {
   if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
   free_all(b.allocs);
   (void)hipFree(b.ring);
-  (void)hipHostFree(b.host);
   ++m->bws_gen;
   b = BatchWs();
-  const size_t staged = static_cast<size_t>(n) * 4 * sizeof(int32_t);
-  if ((e = hipHostMalloc(reinterpret_cast<void**>(&b.host), staged)) != hipSuccess)
-    return hip_fail(e, "hipHostMalloc batch rows");
-  if ((e = hipHostGetDevicePointer(reinterpret_cast<void**>(&b.host_dev), b.host, 0)) != hipSuccess)
-    return hip_fail(e, "hipHostGetDevicePointer batch rows");
   SOC_TRY(dev_alloc_t(b.allocs, n, &b.ids));
   SOC_TRY(dev_alloc_t(b.allocs, n, &b.pos));
   SOC_TRY(dev_alloc_t(b.allocs, n, &b.start));
@@ -1175,17 +1182,31 @@ int enqueue_batch_step(soc_model* m, soc_kv* kv, int n, int max_split, int32_t* 
   return SOC_OK;
 }
 
+// Waits for a batch call's work where the call returns early: its kernels read the context's staged rows, which the next
+// call (of any model) writes.
+struct DrainOnReturn {
+  hipStream_t s;
+  bool drained = false;
+  ~DrainOnReturn() {
+    if (!drained) (void)hipStreamSynchronize(s);
+  }
+};
+
 // Uploads the batch's rows (ids, positions = current lengths, slots) into m->bws: one kernel reads them from pinned
 // memory, and a step's tokens come back through it (four copies from pageable memory and one back were a host wait
-// each: 100 rows of four Qwen3-0.6B layers 603 -> 572 us a call, 16 of Qwen3-4B 502 -> 478).
+// each: 100 rows of four Qwen3-0.6B layers 603 -> 572 us a call, 16 of Qwen3-4B 502 -> 478). The memory is the context's:
+// pinned per model, and again as a batch grew, it cost the first step of a model what it saved (16 rows of four Qwen3-4B
+// layers: 813 -> 761 us).
 int upload_batch(soc_model* m, soc_kv* kv, int n, const int32_t* slots, const int32_t* tokens) {
   BatchWs& b = m->bws;
+  int32_t* host = m->ctx->readback + kReadbackBatch;
   for (int i = 0; i < n; ++i) {
-    b.host[i] = tokens[i];
-    b.host[n + i] = slots[i];
-    b.host[2 * n + i] = kv->len[slots[i]];
+    host[i] = tokens[i];
+    host[n + i] = slots[i];
+    host[2 * n + i] = kv->len[slots[i]];
   }
-  const hipError_t e = soc::launch_stage_batch(b.host_dev, n, b.ids, b.slots, b.pos, b.start, m->ctx->stream);
+  const hipError_t e = soc::launch_stage_batch(m->ctx->readback_dev + kReadbackBatch, n, b.ids, b.slots, b.pos, b.start,
+                                               m->ctx->stream);
   return e == hipSuccess ? SOC_OK : hip_fail(e, "batch rows");
 }
 
@@ -1418,7 +1439,6 @@ int soc_model_destroy(soc_model* m) {
   free_all(m->pws.allocs);
   free_all(m->bws.allocs);
   (void)hipFree(m->bws.ring);
-  (void)hipHostFree(m->bws.host);
   (void)hipFree(m->wbuf);
   (void)hipFree(m->rope_cos);
   (void)hipFree(m->rope_sin);
@@ -2126,18 +2146,6 @@ int soc_prefill(soc_model* m, soc_kv* kv, int32_t slot, const int32_t* ids, int3
 namespace {
 // One decode step of one slot (the checks done by the caller): token `last`, or the id at dev_last in device memory;
 // logits [V] nullable (host or device), one synchronisation.
-int ensure_readback(soc_ctx* ctx) {
-  if (ctx->readback != nullptr) return SOC_OK;
-  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&ctx->readback), 64);
-  if (e != hipSuccess) return hip_fail(e, "hipHostMalloc readback words");
-  if ((e = hipHostGetDevicePointer(reinterpret_cast<void**>(&ctx->readback_dev), ctx->readback, 0)) != hipSuccess) {
-    (void)hipHostFree(ctx->readback);
-    ctx->readback = nullptr;
-    return hip_fail(e, "hipHostGetDevicePointer");
-  }
-  return SOC_OK;
-}
-
 int decode_one(soc_model* m, soc_kv* kv, int32_t slot, int32_t last, const int32_t* dev_last, float* logits,
                int32_t* next_token) {
   SOC_TRY(ensure_decode_ws(m, kv->cap));
@@ -2395,9 +2403,10 @@ int soc_decode_batch(soc_model* m, soc_kv* kv, int32_t n, const int32_t* slots, 
   SOC_TRY(validate_batch(m, kv, n, slots, tokens, 1, &max_len));
   SOC_TRY(ensure_prefill_ws(m, n, max_len, n));
   SOC_TRY(ensure_batch_ws(m, n));
+  DrainOnReturn drain{m->ctx->stream};
   SOC_TRY(upload_batch(m, kv, n, slots, tokens));
-  SOC_TRY(enqueue_batch_step(m, kv, n, (max_len + kAttnChunk - 1) / kAttnChunk,
-                             m->bws.host_dev + static_cast<size_t>(3) * m->bws.cap, 1));
+  constexpr size_t kTokens = kReadbackBatch + static_cast<size_t>(3) * kMaxBatchRows;  // on their way out
+  SOC_TRY(enqueue_batch_step(m, kv, n, (max_len + kAttnChunk - 1) / kAttnChunk, m->ctx->readback_dev + kTokens, 1));
   hipStream_t s = m->ctx->stream;
   hipError_t e;
   if (logits != nullptr &&
@@ -2405,7 +2414,8 @@ int soc_decode_batch(soc_model* m, soc_kv* kv, int32_t n, const int32_t* slots, 
                           s)) != hipSuccess)
     return hip_fail(e, "hipMemcpyAsync logits");
   if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "decode batch");
-  std::memcpy(next_tokens, m->bws.host + static_cast<size_t>(3) * m->bws.cap, static_cast<size_t>(n) * 4);
+  drain.drained = true;
+  std::memcpy(next_tokens, m->ctx->readback + kTokens, static_cast<size_t>(n) * 4);
   for (int i = 0; i < n; ++i) kv->len[slots[i]] += 1;
   return SOC_OK;
   SOC_API_END
@@ -2423,6 +2433,7 @@ int soc_decode_batch_steps(soc_model* m, soc_kv* kv, int32_t n, const int32_t* s
   if (steps == 0) return SOC_OK;
   SOC_TRY(ensure_prefill_ws(m, n, kv->cap, n));
   SOC_TRY(ensure_batch_ws(m, n));
+  DrainOnReturn drain{m->ctx->stream};
   SOC_TRY(upload_batch(m, kv, n, slots, tokens));
   hipStream_t s = m->ctx->stream;
   BatchWs& b = m->bws;
@@ -2473,6 +2484,7 @@ int soc_decode_batch_steps(soc_model* m, soc_kv* kv, int32_t n, const int32_t* s
   if ((e = hipMemcpyAsync(host.data(), ring, host.size() * 4, hipMemcpyDeviceToHost, s)) != hipSuccess)
     return hip_fail(e, "hipMemcpyAsync tokens");
   if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "decode batch steps");
+  drain.drained = true;
   for (int t = 0; t < steps; ++t)
     for (int i = 0; i < n; ++i) tokens_out[static_cast<size_t>(t) * n + i] = host[static_cast<size_t>(i) * steps + t];
   for (int i = 0; i < n; ++i) kv->len[slots[i]] += steps;

@@ -319,3 +319,32 @@ def test_batch_row_gemm_edges(gpu_ctx, n):
         for kv in kvs:
             kv.close()
         m.close()
+
+
+def test_batch_rows_of_models_that_share_a_context(gpu_ctx):
+    """Two models of one context take turns with growing and shrinking batches (their rows are staged in the same pinned
+    words): each call's logits and tokens are bit for bit those of the model stepping alone."""
+    cfgs = [small_cfg(), S.QwenConfig(vocab_size=64, hidden_size=128, num_hidden_layers=1, num_attention_heads=2,
+                                      num_key_value_heads=1, intermediate_size=128, tie_word_embeddings=True)]
+    models = [S.Model(gpu_ctx, c).load(S.synth_weights(c, 90 + i)) for i, c in enumerate(cfgs)]
+    counts = (3, 1, 40, 17, 1024, 2)
+    kvs = [S.KVCache(m, max(counts), 8) for m in models for _ in range(2)]
+
+    def step(which, turn, copy):
+        n, kv = counts[turn], kvs[2 * which + copy]
+        rng = np.random.default_rng(10 * turn + which)
+        slots = rng.permutation(max(counts))[:n].astype(np.int32)
+        return S.decode_batch(models[which], kv, slots, rng.integers(0, cfgs[which].vocab_size, n).astype(np.int32))
+
+    try:
+        alone = [[step(i, t, 0) for t in range(len(counts))] for i in range(2)]
+        for t in range(len(counts)):
+            for i in range(2):
+                lg, nxt = step(i, t, 1)
+                assert np.array_equal(lg, alone[i][t][0]) and np.array_equal(nxt, alone[i][t][1]), (t, i)
+                assert np.array_equal(nxt, np.argmax(lg, axis=1))
+    finally:
+        for kv in kvs:
+            kv.close()
+        for m in models:
+            m.close()
