@@ -362,30 +362,15 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int qpos, Att
   }
   __syncthreads();
   // a wave per head, a lane per chunk (one thread walking 64 chunks' maxima and exponentials took as long as the
-  // chunk itself); the sums in chunk order, from LDS
+  // chunk itself)
   for (int j = wid; j < G; j += 4) {
     float M = -INFINITY;
     for (int t = lane; t < nact; t += 64) M = fmaxf(M, cm[j][t]);
     M = wave_max(M);
     for (int t = lane; t < nact; t += 64) cm[j][t] = expf(cm[j][t] - M);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the sums read the other lanes' weights
-    __builtin_amdgcn_wave_barrier();
-    float L = 0.0f;
-    for (int t0 = 0; t0 < nact; t0 += 8) {
-      float e[8], l[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int t = min(t0 + u, nact - 1);
-        e[u] = cm[j][t];
-        l[u] = cl[j][t];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (t0 + u < nact) L = fmaf(l[u], e[u], L);
-    }
-    if (lane == 0) lstat[j] = L;
   }
   __syncthreads();
+  // both sums in chunk order, the weights' beside the values' in every thread
 #pragma unroll
   for (int q = 0; q < OPT; ++q) {
     const int idx = tid + 256 * q;
@@ -393,19 +378,25 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int qpos, Att
     const int j = idx / HD, i = idx % HD;
     const float* p0 = a.part + (static_cast<size_t>(b) * a.nq + g * G + j) * a.max_split * stride + i;
     const float* ej = cm[j];
-    float O = 0.0f;
+    float O = 0.0f, L = 0.0f;
 #pragma unroll
     for (int u = 0; u < 16; ++u)
-      if (u < nact) O += v0[q][u] * ej[u];
+      if (u < nact) {
+        O += v0[q][u] * ej[u];
+        L += cl[j][u] * ej[u];
+      }
     for (int t = 16; t < nact; t += 16) {
       float v[16];
 #pragma unroll
       for (int u = 0; u < 16; ++u) v[u] = ld_dev(p0 + min(t + u, nact - 1) * stride);
 #pragma unroll
       for (int u = 0; u < 16; ++u)
-        if (t + u < nact) O += v[u] * ej[t + u];
+        if (t + u < nact) {
+          O += v[u] * ej[t + u];
+          L += cl[j][t + u] * ej[t + u];
+        }
     }
-    put(j, i, O / lstat[j]);
+    put(j, i, O / L);
   }
   if (tid == 0) st_dev(a.counters + b * a.nkv + g, 0);
 }
