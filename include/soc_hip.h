@@ -138,7 +138,9 @@ int soc_quantize_group(const uint16_t* w, int64_t n, int64_t k, int32_t bits, vo
 /* Packs every projection of a finalized model (q/k/v, o, gate/up, down) with soc_quantize_group; afterwards prefill
  * and decode run those projections as group-quantized matmuls (soc_qmm's kernels) on fp16 activation rows, with
  * the embedding, norms, attention and LM head unchanged. Quantized models decode on the per-operator path (no
- * one-launch kernels) and do not support the ragged batch. No counterpart in the reference. */
+ * one-launch kernels) and do not support the ragged batch. A prompt of 2 to 8 rows sums in another order than one row
+ * does, and a longer one runs on the weights rounded to fp16: the same position's logits agree within the rounding of
+ * the fp16 activation rows (about 7e-4), not bit for bit. No counterpart in the reference. */
 int soc_model_quantize(soc_model* model, int32_t bits);
 /* Bytes of weights held on the device. */
 int soc_model_weight_bytes(const soc_model* model, int64_t* bytes);
@@ -224,7 +226,9 @@ int soc_decode_steps_noalloc(soc_model* model, soc_kv* kv, int32_t slot, int32_t
  *      DecodeNextToken, Mac/gpu/src/runtime/generation_context.cpp:68-172, one token at pos = len - 1); a batch of n
  *      rows gives each row exactly that semantics for its own slot, in one pass over the weights: row i feeds
  *      tokens[i] to slot slots[i] at position = that slot's current length (per-sequence KV length, any mix of
- *      lengths) and appends its K/V. Slots must be distinct; 1 <= n <= 1024. ---- */
+ *      lengths) and appends its K/V. Slots must be distinct; 1 <= n <= 1024. A row's result does not depend on the
+ *      other rows or its place among them; the order of its fp32 sums follows the range that n lies in (1 .. 16, 17 ..
+ *      64, then steps of 128 rows from 65), so its last bits may differ from one range to the next. ---- */
 /* One step. logits: nullable [n][vocab]; next_tokens [n]: greedy ids (lowest index on ties, sampler.cpp:42-48). */
 int soc_decode_batch(soc_model* model, soc_kv* kv, int32_t n, const int32_t* slots, const int32_t* tokens,
                      float* logits, int32_t* next_tokens);
@@ -261,7 +265,8 @@ int soc_attention_prefill(soc_ctx* ctx, const float* q, const void* keys, const 
  * Mac/gpu/src/module/qwen_attention.mm): q fp32 [nq * 128], out fp32 [nq * 128]. */
 int soc_attention_decode(soc_ctx* ctx, const float* q, const void* keys, const void* values, float* out,
                          int32_t kv_len, int32_t nq, int32_t nkv, int32_t head_dim, int32_t cap);
-/* Group-quantized matmul: y[M][N] = x[M][K] . dequant(codes, scales)^T; bits 8 or 4; group 64 along K. */
+/* Group-quantized matmul: y[M][N] = x[M][K] . dequant(codes, scales)^T; bits 8 or 4; group 64 along K. The kernel
+ * follows M, N and K: a row's sums, all fp32 of exact products, have another order at another M. */
 int soc_qmm(soc_ctx* ctx, const void* x_f16, const void* codes, int32_t bits, const void* scales_f16, float* y,
             int32_t m, int32_t n, int32_t k);
 /* Dequantize to fp32 [N][K] (bit-exact contract: w = float(code) * float(scale)). */

@@ -693,9 +693,14 @@ constexpr int kRowsSlots = 512;  // two 128 x 128 blocks per CU
 struct RowsPlan {
   int bm, splits;
 };
-RowsPlan rows_plan(int M, int N, int K) {
-  const int bm = M <= 64 ? 64 : 128;
-  const int tiles = ((M + bm - 1) / bm) * ((N + 127) / 128), slices = K / 32;
+// The splits are planned for whole row tiles (up to 64 rows, 128, 256, 384 ..): within one of these ranges a row's sums
+// have one order, and its bits do not change as other sequences join or leave (planned for the very row count, the
+// split of Qwen3-0.6B's o projection went from 32 to 16 between 17 and 64 rows, at no gain: two layers and a 16384-word
+// head at 17, 24, 65, 100 and 257 rows, us, whole tiles against the row count: Qwen3-0.6B 142 : 144, 145 : 148, 171 : 173,
+// 188 : 186, 278 : 274, Qwen3-4B 262 : 261, 268 : 266, 325 : 325, 351 : 351, 626 : 625).
+RowsPlan rows_plan(int rows, int N, int K) {
+  const int bm = rows <= 64 ? 64 : 128, M = (rows + bm - 1) / bm * bm;
+  const int tiles = M / bm * ((N + 127) / 128), slices = K / 32;
   int best = 1;
   double cost = 0.0;
   for (int sp = 1; sp <= slices && sp <= 32 && (sp == 1 || tiles * sp <= kRowsSlots); ++sp) {

@@ -1,6 +1,7 @@
 // rows_epi.hip - the second half of a ragged decode batch's projections beyond 16 rows: the split-K partial sums that
 // launch_gemm_rows leaves ([split][row][N], fp32) added in split order, and what follows the projection in the layer.
-// A row's result never depends on the other rows. Bound by the partials' round trip (they stay in L2 and the
+// A row's result does not depend on what the other rows hold or where they stand; the number of splits, and with it the
+// order of a row's sums, follows the number of row tiles (rows_plan in gemm.hip). Bound by the partials' round trip (they stay in L2 and the
 // memory-side cache) and the launch; every load of a thread's sums goes out before the first add.
 #include "kernels.h"
 

@@ -961,7 +961,7 @@ int ensure_readback(soc_ctx* ctx) {
 }
 
 // A batch step's projections: the skinny kernels (input RMSNorm, q/k norm, RoPE and KV append folded in) up to their 16
-// rows, else the split-K row GEMMs, which stream the weights once whatever the rows (two layers and a 16384-word head,
+// rows, else the split-K row GEMMs, which stream the weights once per 128 rows (two layers and a 16384-word head,
 // us per step, against skinny slabs of 16: Qwen3-0.6B 17 rows 198 : 277, 64 rows 226 : 470; Qwen3-4B 17 rows 329 : 400,
 // 64 rows 374 : 703).
 bool batch_skinny_path(const soc_model* m, int n) { return m->pws.skpart != nullptr && n <= 16; }

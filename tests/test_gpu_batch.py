@@ -61,9 +61,8 @@ def test_batch_rows_equal_single_sequence_decode(gpu_ctx, nq, nkv):
 
 
 def test_batch_many_rows_slabs_and_tiled_path(gpu_ctx):
-    """20 rows (two 16-row slabs of the skinny projection) and 70 rows (the tiled GEMM on the same pre-split
-    activations): every row agrees with single-sequence decode of its slot within the model tolerance, with the
-    same greedy token."""
+    """20 and 70 rows, beyond the 16 of the skinny projections (split-K row GEMMs on 64- and 128-row tiles): every row
+    agrees with single-sequence decode of its slot within the model tolerance, with the same greedy token."""
     cfg = small_cfg()
     m = S.Model(gpu_ctx, cfg).load(S.synth_weights(cfg, 33))
     nslots = 70
@@ -348,3 +347,30 @@ def test_batch_rows_of_models_that_share_a_context(gpu_ctx):
             kv.close()
         for m in models:
             m.close()
+
+
+@pytest.mark.parametrize("hidden,inter,nq", [(1024, 3072, 16), (2560, 9728, 32)])
+def test_batch_rows_keep_their_bits_as_others_join(gpu_ctx, hidden, inter, nq):
+    """A sequence's logits and appended keys are bit for bit the same at every row count that takes as many row tiles: 1 ..
+    16 rows, 17 .. 64, 65 .. 128, 129 .. 256 (Qwen3-0.6B and 4B widths, where K is split)."""
+    cfg = S.QwenConfig(vocab_size=512, hidden_size=hidden, num_hidden_layers=1, num_attention_heads=nq,
+                       num_key_value_heads=8, intermediate_size=inter, tie_word_embeddings=True)
+    m = S.Model(gpu_ctx, cfg).synthesize(7)
+    kv = S.KVCache(m, 256, 48)
+    toks = np.random.default_rng(8).integers(0, cfg.vocab_size, 256).astype(np.int32)
+    try:
+        for slot in range(256):
+            kv.fill_synthetic(slot, 1 + slot % 40, 9)
+        for counts in ((1, 2, 9, 16), (17, 18, 33, 64), (65, 100, 128), (129, 200, 256)):
+            first = None
+            for n in counts:
+                for slot in range(n):
+                    S.capi.check(S.lib().soc_kv_set_length(kv.h, slot, 1 + slot % 40))
+                rows = np.arange(n, dtype=np.int32)
+                lg, _ = S.decode_batch(m, kv, rows, toks[:n])
+                got = lg[: counts[0]], kv.read(0, 0)[0]
+                first = first or got
+                assert np.array_equal(got[0], first[0]) and np.array_equal(got[1], first[1]), n
+    finally:
+        kv.close()
+        m.close()
