@@ -138,9 +138,9 @@ int soc_quantize_group(const uint16_t* w, int64_t n, int64_t k, int32_t bits, vo
 /* Packs every projection of a finalized model (q/k/v, o, gate/up, down) with soc_quantize_group; afterwards prefill
  * and decode run those projections as group-quantized matmuls (soc_qmm's kernels) on fp16 activation rows, with
  * the embedding, norms, attention and LM head unchanged. Quantized models decode on the per-operator path (no
- * one-launch kernels) and do not support the ragged batch. A prompt of 2 to 8 rows sums in another order than one row
- * does, and a longer one runs on the weights rounded to fp16: the same position's logits agree within the rounding of
- * the fp16 activation rows (about 7e-4), not bit for bit. No counterpart in the reference. */
+ * one-launch kernels) and do not support the ragged batch. A prompt of 1, 2, 3 or 4, and 5 to 8 rows each sums in an
+ * order of its own, and a longer one runs on the weights rounded to fp16: the same position's logits agree within the
+ * rounding of the fp16 activation rows (about 7e-4), not bit for bit. No counterpart in the reference. */
 int soc_model_quantize(soc_model* model, int32_t bits);
 /* Bytes of weights held on the device. */
 int soc_model_weight_bytes(const soc_model* model, int64_t* bytes);
@@ -228,7 +228,7 @@ int soc_decode_steps_noalloc(soc_model* model, soc_kv* kv, int32_t slot, int32_t
  *      tokens[i] to slot slots[i] at position = that slot's current length (per-sequence KV length, any mix of
  *      lengths) and appends its K/V. Slots must be distinct; 1 <= n <= 1024. A row's result does not depend on the
  *      other rows or its place among them; the order of its fp32 sums follows the range that n lies in (1 .. 16, 17 ..
- *      64, then steps of 128 rows from 65), so its last bits may differ from one range to the next. ---- */
+ *      64, 65 .. 128, 129 .. 256, then every 128 rows), so its last bits may differ from one range to the next. ---- */
 /* One step. logits: nullable [n][vocab]; next_tokens [n]: greedy ids (lowest index on ties, sampler.cpp:42-48). */
 int soc_decode_batch(soc_model* model, soc_kv* kv, int32_t n, const int32_t* slots, const int32_t* tokens,
                      float* logits, int32_t* next_tokens);

@@ -374,3 +374,60 @@ def test_batch_rows_keep_their_bits_as_others_join(gpu_ctx, hidden, inter, nq):
     finally:
         kv.close()
         m.close()
+
+
+def _first_token_logits(cfg, w, toks, cached, round_head=False):
+    """Logits of sequences of one token in float64; the attention, over one key, returns its value, for which the cached
+    fp16 values [layers][n][kv heads * 128] stand. round_head: the head's input rounded to fp16, as it would be without
+    its low half. Also the values before their rounding."""
+    f = {k: v.view(np.float16).astype(np.float64) for k, v in w.items()}
+
+    def norm(x, gain):
+        return x / np.sqrt(np.mean(x * x, -1, keepdims=True) + cfg.rms_norm_eps) * gain
+
+    x, values = f["model.embed_tokens.weight"][toks], []
+    for l in range(cfg.num_hidden_layers):
+        p = f"model.layers.{l}."
+        values.append(norm(x, f[p + "input_layernorm.weight"]) @ f[p + "self_attn.v_proj.weight"].T)
+        v = cached[l].astype(np.float64).reshape(len(toks), -1, 128)
+        attn = np.repeat(v, cfg.num_attention_heads // cfg.num_key_value_heads, axis=1).reshape(len(toks), -1)
+        x = x + attn @ f[p + "self_attn.o_proj.weight"].T
+        h = norm(x, f[p + "post_attention_layernorm.weight"])
+        g = h @ f[p + "mlp.gate_proj.weight"].T
+        x = x + (g / (1 + np.exp(-g)) * (h @ f[p + "mlp.up_proj.weight"].T)) @ f[p + "mlp.down_proj.weight"].T
+    h = norm(x, f["model.norm.weight"])
+    if round_head:
+        h = h.astype(np.float16).astype(np.float64)
+    return h @ f["model.embed_tokens.weight"].T, np.stack(values)
+
+
+@pytest.mark.parametrize("n,hidden,vocab", [
+    (65, 256, 65537), (130, 256, 65537),             # the head's 128 x 128 tiles (512 of them), one and two high
+    (17, 1024, 512), (65, 2048, 512), (17, 2560, 512), (130, 4160, 512),  # each width of the residual and norm step
+])
+def test_batch_row_gemms_in_full_precision(gpu_ctx, n, hidden, vocab):
+    """Rows beyond 16 against a float64 forward, tightly enough to see the low halves of the activation pairs: fp32 sums
+    and 22-bit activations are good for some 1e-6 of a row's norm (2e-7 to 7e-7 seen), the head's input without its low
+    half is off by 2^-11 / sqrt(12) = 1.4e-4 (checked on the reference). The cached values are the reference's to within
+    one fp16 rounding."""
+    cfg = S.QwenConfig(vocab_size=vocab, hidden_size=hidden, num_hidden_layers=2, num_attention_heads=4,
+                       num_key_value_heads=2, intermediate_size=512, tie_word_embeddings=True)
+    w = S.synth_weights(cfg, 61, 0.05)
+    m = S.Model(gpu_ctx, cfg).load(w)
+    kv = S.KVCache(m, n, 4)
+    try:
+        toks = np.random.default_rng(62).integers(0, vocab, n).astype(np.int32)
+        lg, _ = S.decode_batch(m, kv, np.arange(n, dtype=np.int32), toks)
+        cached = np.stack([[kv.read(slot, l)[1][:, 0].reshape(-1) for slot in range(n)]
+                           for l in range(cfg.num_hidden_layers)])
+    finally:
+        kv.close()
+        m.close()
+    ref, values = _first_token_logits(cfg, w, toks, cached)
+    # half an fp16 step, and 3e-6 of a value's spread over the row (0.05 sqrt(hidden) <= 3.3) for its fp32 sum
+    assert np.all(np.abs(cached - values) <= 2.0 ** -11 * np.abs(values) + 1e-5)
+    scale = np.linalg.norm(ref, axis=1)
+    err = np.max(np.linalg.norm(lg - ref, axis=1) / scale)
+    rounded = np.min(np.linalg.norm(_first_token_logits(cfg, w, toks, cached, True)[0] - ref, axis=1) / scale)
+    print(f"[rows] {n} x {hidden}, {vocab} words: {err:.2e}, head input in fp16 alone {rounded:.2e}", flush=True)
+    assert err <= 1e-5 < rounded / 2, (err, rounded)

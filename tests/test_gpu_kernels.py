@@ -143,3 +143,23 @@ def test_qmm_row_kernels_match_oracle(gpu_ctx, oracle_mod, bits, m, n, k):
     finally:
         for p in (dc, ds, dx, dx1, dy):
             ctx.free(p)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("n,k", [(1000, 6144), (17, 7104), (48, 10176)])
+@pytest.mark.parametrize("m", [2, 4])
+def test_qmm_row_kernels_long_rows(gpu_ctx, oracle_mod, bits, m, n, k):
+    """soc_qmm on rows beyond what k_qrows holds of them in registers (K > 5120 int4, > 4096 int8): several passes over K
+    per tile, the last one partly filled, within the summation bound."""
+    ctx = gpu_ctx
+    codes, scales, x = _qmm_inputs(n, k, bits, m)
+    ref = oracle_mod.qmm_group(x, codes, bits, scales, k, n)
+    bound = _err_bound(x.view(np.float16).astype(np.float32), oracle_mod.dequant_group(codes, bits, scales, n, k))
+    dc, ds, dy, dx = ctx.upload(codes), ctx.upload(scales), ctx.alloc(m * n * 4), ctx.upload(x)
+    try:
+        S.qmm(ctx, dx, dc, bits, ds, dy, m, n, k)
+        y = ctx.download(dy, (m, n), np.float32)
+        assert np.all(np.abs(y - ref) <= bound), float(np.max(np.abs(y - ref) - bound))
+    finally:
+        for p in (dc, ds, dx, dy):
+            ctx.free(p)

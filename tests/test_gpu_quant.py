@@ -112,3 +112,26 @@ def test_quantized_decode_keeps_its_bits(gpu_ctx, golden, bits, length):
         m.close()
     want = golden("qdecode_rows.npz")[f"int{bits}_{length}"]
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), float(np.max(np.abs(got - want)))
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("n", [2, 3, 5, 8])
+@pytest.mark.parametrize("hidden,inter", [(1088, 6144), (4160, 1088)])
+def test_quantized_long_rows(gpu_ctx, oracle_mod, bits, n, hidden, inter):
+    """Prompts of 2 to 8 rows where a projection's rows outgrow the registers of the row kernel (K > 4096 int4, 3072
+    int8), so that each tile takes several passes over K: the residual form (inter 6144, the down projection of
+    Qwen3-1.7B), the RMSNorm and SwiGLU forms (hidden 4160), against the oracle on the dequantized weights."""
+    cfg = S.QwenConfig(vocab_size=512, hidden_size=hidden, num_hidden_layers=1, num_attention_heads=4,
+                       num_key_value_heads=2, intermediate_size=inter, tie_word_embeddings=True)
+    w = S.synth_weights(cfg, 47, 0.05)
+    m = S.Model(gpu_ctx, cfg).load(w).quantize(bits)
+    om = oracle_mod.OracleModel(cfg, _dequantized(oracle_mod, w, bits))
+    kv = S.KVCache(m, 1, 16)
+    try:
+        ids = S.synth_tokens(48, "long rows", cfg.vocab_size, n)
+        lg, _ = S.prefill(m, kv, 0, ids, 0, logit_rows=n)
+        ref = oracle_mod.OracleCache(om, 16).forward(ids, 0, logit_rows=n)
+        assert_logits_close(lg, ref, f"int{bits} {hidden}/{inter}, {n} rows")
+    finally:
+        kv.close()
+        m.close()
