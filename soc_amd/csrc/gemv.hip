@@ -313,14 +313,15 @@ __global__ __launch_bounds__(256) void k_lm_head_argmax(LmHeadArgs a) {
 // dequant_group's contract). BITS = 8: codes int8 [N][K]; BITS = 4: two's complement nibbles, even k in the low nibble,
 // [N][K/2].
 //
-// k_qmm (two rows of tall matrices, and operands off 16-byte alignment): each lane streams 16-byte chunks of a row's codes (16 int8 or 32 int4 codes; a
-// chunk never crosses a scale group). The codes become exact fp16 pairs without per-code conversions: the biased code
-// (code + 128, or the nibble + 8) is placed in the low mantissa bits of 1024.0 (fp16 0x64xx) by one byte permute (int8)
-// or one mask-xor (int4), and one packed fp16 subtract of 1152 (or 1032) leaves the code itself (int4 nibbles in bits
-// 4..7: one packed fma by 1/16 minus 72, so that half the nibbles need no shift). v_dot2_f32_f16 then accumulates code
-// pairs times fp16 activation pairs in fp32 (products exact), and one fma per chunk applies the group scale. The
-// activations are staged once per block in LDS as fp16 pairs in the order the codes unpack (int4: k and k + 4 of each
-// group of 8). L lanes share a row (64, or 32 / 16 for short rows) and each lane keeps RR rows in flight.
+// k_qmm (two rows of tall matrices, and operands off 16-byte alignment): each lane streams 16-byte chunks of a row's
+// codes (16 int8 or 32 int4 codes; a chunk never crosses a scale group). The codes become exact fp16 pairs without
+// per-code conversions: the biased code (code + 128, or the nibble + 8) is placed in the low mantissa bits of 1024.0
+// (fp16 0x64xx) by one byte permute (int8) or one mask-xor (int4), and one packed fp16 subtract of 1152 (or 1032) leaves
+// the code itself (int4 nibbles in bits 4..7: one packed fma by 1/16 minus 72, so that half the nibbles need no shift).
+// v_dot2_f32_f16 then accumulates code pairs times fp16 activation pairs in fp32 (products exact), and one fma per
+// chunk applies the group scale. The activations are staged once per block in LDS as fp16 pairs in the order the codes
+// unpack (int4: k and k + 4 of each group of 8). L lanes share a row (64, or 32 / 16 for short rows) and each lane
+// keeps RR rows in flight.
 namespace {
 typedef _Float16 qh2 __attribute__((ext_vector_type(2)));
 typedef _Float16 sk_qh8 __attribute__((ext_vector_type(8)));

@@ -49,8 +49,8 @@ struct QmmArgs {
   int M, N, K;
 };
 hipError_t launch_qmm(const QmmArgs& a, int bits, hipStream_t s);
-// The same products for 1 <= M <= 8 rows on matrix cores, with a decode projection's neighbours fused in
-// (qrows.hip). Activations: xh (fp16 [M][K]), or x (fp32, rounded to fp16), or RMSNorm(x) with `gain` (rounded).
+// The same products for 1 <= M <= 8 rows (one row of K <= 16384 on the vector ALUs, else matrix cores), with a decode
+// projection's neighbours fused in (qrows.hip). Activations: xh (fp16 [M][K]), or x (fp32, rounded to fp16), or RMSNorm(x) with `gain` (rounded).
 //   EPI_STORE: y = sums (xh, or x with gain). EPI_RESIDUAL: y += sums (xh, or x without gain). EPI_SWIGLU: rows
 //   [0, N / 2) are gate and [N / 2, N) up: yh [M][N / 2] = fp16(silu(gate) * up) (x with gain).
 struct QRowsArgs {

@@ -76,7 +76,8 @@ __global__ __launch_bounds__(512, XF == QX_F16 && KW == 8 && !LONG && UW * BITS 
 k_qrows(QRowsArgs a) {
   constexpr int TW = 8 / KW;               // tiles side by side
   constexpr int TS = 4 / TW;               // tiles one after the other between barriers
-  constexpr bool AHEAD = !(BITS == 8 && UW == 6 && !LONG && XF == QX_F16);  // registers, see below
+  // the next tile's codes requested a tile ahead, but where holding both spills (24 of 128 registers: int8, UW = 6)
+  constexpr bool AHEAD = !(BITS == 8 && UW == 6 && !LONG && XF == QX_F16);
   static_assert(KW == 8 || (XF == QX_F16 && EPI == EPI_STORE && !LONG && KW >= 2), "wave groups");
   constexpr int GPU = BITS == 4 ? 2 : 1;   // scale groups per unit
   constexpr int KU = 64 * GPU;             // codes of a row per unit

@@ -28,6 +28,11 @@ Fixtures:
                     the slot, length, token, 64 largest logits, logits at 512 seeded indices and argmax, from the
                     compiled reference.
 
+One file is not written here, since no reference has its arithmetic: qdecode_rows.npz, logits of four greedy-decode steps
+of int4 and int8 models (two layers of Qwen3-0.6B widths, weights seed 81, 97 and 300 cached keys seed 82, tokens 11,
+200, 77, 5) as this library gave them with a kernel each for norm, projection, SwiGLU and residual. The fused kernels are
+held to those bits; the values are held to the oracle elsewhere (tests/test_gpu_quant.py).
+
 Usage: python tests/golden/make_golden.py [--skip-0p6b] [--only NAME[,NAME...]]
        (names: dtype, ops, quant, small, 0p6b, 0p6b_s2, prefill2048, ragged4b)
 """

@@ -82,8 +82,8 @@ def _qmm_inputs(n, k, bits, m):
 @pytest.mark.parametrize("mode,m", [("auto", 1), ("auto", 2), ("auto", 4), ("auto", 8),
                                     ("mfma", 2), ("mfma", 4), ("mfma", 8)])
 def test_qmm_matches_oracle(gpu_ctx, oracle_mod, monkeypatch, bits, m, n, k, mode):
-    """auto: the dot-product kernel at m = 1 and for short matrices, the MFMA kernel for tall ones at m >= 2;
-    mfma: the MFMA kernel wherever it applies (it serves m >= 2)."""
+    """auto: the kernel that soc_qmm takes for the shape (one row's dot products, the row kernels for 2 to 8, the MFMA
+    kernel for tall matrices at m >= 2); mfma: the MFMA kernel wherever it applies (it serves m >= 2)."""
     if mode == "mfma":
         monkeypatch.setenv("SOC_QMM", "mfma")
     ctx = gpu_ctx
